@@ -35,6 +35,10 @@
 // 8 g .. 8 g + 7, exactly the B operand of O^T += V^T P^T.  Online softmax in
 // the log2 domain with the lazily moved maximum of the other kernels; l sums
 // the bf16-rounded p that the P.V product multiplies.
+//
+// Head dims 256 and 512 without per-key masks run attn_hilo32_kernel (32-row
+// waves); this kernel takes head dims up to 128, head dims below their tile
+// and MASK_KEYS.
 #include "attn_common.hpp"
 
 #include <limits.h>
@@ -431,6 +435,7 @@ hipError_t launch_hilo_hd(const LaunchPlan& p, const AttnArgs& a, hipStream_t st
 int hilo_rows() { return HiloGeom<256>::QROWS; }
 
 hipError_t launch_hilo(const LaunchPlan& p, const AttnArgs& a, hipStream_t st) {
+    if (!p.w16) return launch_hilo32(p, a, st);
     if (a.hd > p.hd_tile) return hipErrorInvalidValue;
     for (int i = 0; i < a.n_batch; ++i)
         if (!a.slot[i].klo || !a.slot[i].vlo) return hipErrorInvalidValue;  // no lo planes

@@ -1178,21 +1178,24 @@ static dr::LaunchPlan plan_hilo(dr_ctx* ctx, const dr::AttnArgs& a, int hd, int 
     dr::LaunchPlan p{};
     p.hd_tile = hd_tile_for((size_t)hd);
     p.block_n = 32;
-    p.rb = dr::hilo_rows() / 32;
+    // 32-row waves (attn_hilo32_kernel) at the head dims and masks they are
+    // built for, else the 16-row kernel
+    const bool w32 = dr::hilo32_rows(p.hd_tile) > 0 && hd == p.hd_tile && mask != dr::MASK_KEYS;
+    const int rows = w32 ? dr::hilo32_rows(p.hd_tile) : dr::hilo_rows();
+    p.rb = rows / 32;
     p.kq = 1;
-    p.waves = p.hd_tile > 256 ? 8 : 4;
+    p.waves = !w32 && p.hd_tile > 256 ? 8 : 4;
     p.stages = 1;
-    p.rowgroups = (a.group * max_nq + dr::hilo_rows() - 1) / dr::hilo_rows();
+    p.rowgroups = (a.group * max_nq + rows - 1) / rows;
     p.mask = mask;
-    p.w16 = true;
+    p.w16 = !w32;
     p.kernel = dr::KERNEL_HILO;
     const int base = a.n_batch * a.n_head_kv * p.rowgroups;
     const int ntiles = std::max(1, (max_nk + 31) / 32);
-    // Workgroups that run at once: up to head dim 256 a workgroup takes 64 KB
-    // of LDS or less, so two share a CU, and key splits fill both (C5's
-    // global layer at scale 1.0: 74.8 us at 8 splits against 94.8 at 4; its
-    // sliding layer 46.5 against 49.0).  At 512 (144 KB) one per CU.
-    const int slots = ctx->n_cu * (p.hd_tile > 256 ? 1 : 2);
+    // Workgroups that run at once: the 16-row kernel takes at most 64 KB of
+    // LDS up to head dim 256, so two share a CU and key splits fill both; the
+    // others take a CU each.
+    const int slots = ctx->n_cu * (w32 || p.hd_tile > 256 ? 1 : 2);
     int split = 1;
     if (ctx->force_split > 0)
         split = ctx->force_split;
@@ -1219,15 +1222,17 @@ static dr::LaunchPlan plan_for(dr_ctx* ctx, const dr::AttnArgs& a, int hd, int m
                               ctx->merge_in_kernel != 0, a.key_band);
 }
 
-// The hi/lo kernel reads plain Q: with a Q epilogue (bias, QK-norm, RoPE),
-// each batch slot's Q is copied into a workspace and the epilogue
+// The 16-row hi/lo kernel reads plain Q: with a Q epilogue (bias, QK-norm,
+// RoPE), each batch slot's Q is copied into a workspace and the epilogue
 // (qkv_epilogue.hip, Q heads only) runs there first.  Bytes of that
 // workspace (0: the kernel reads the caller's rows): the QK-norm alone at a
 // full head-dim tile needs none, the kernel applies it as it loads Q (a
 // row's sum of squares over four lanes of one wave, or of the row block's
-// two waves at hd 512).
+// two waves at hd 512).  The 32-row kernel applies all three as it loads Q
+// when the rotary covers the head.
 static size_t hilo_q_bytes(const dr::AttnArgs& a, const dr::LaunchPlan& p) {
     if (p.kernel != dr::KERNEL_HILO || (!a.qn_w && !a.qb && !a.rope)) return 0;
+    if (!p.w16 && (!a.rope || a.rot == a.hd)) return 0;
     if (!a.qb && !a.rope && a.hd == p.hd_tile) return 0;
     size_t total = 0;
     for (int b = 0; b < a.n_batch; ++b) total += (size_t)a.slot[b].nq * a.n_head * a.hd;

@@ -376,6 +376,8 @@ bool ring_waves_built(int hd, int waves);
 int ring_merge_splits(int hd);  // most key splits attn_ring_kernel merges in-kernel
 hipError_t launch_hilo(const LaunchPlan& p, const AttnArgs& a, hipStream_t st);
 int hilo_rows();  // query rows per workgroup of attn_hilo_kernel
+hipError_t launch_hilo32(const LaunchPlan& p, const AttnArgs& a, hipStream_t st);
+int hilo32_rows(int hd_tile);  // the same of attn_hilo32_kernel (0: head dim not built)
 hipError_t launch_store(int hd_tile, const StoreArgs& a, hipStream_t st);
 hipError_t launch_gather(int hd_tile, const GatherArgs& a, hipStream_t st);
 hipError_t launch_epilogue(const EpiArgs& a, hipStream_t st);
