@@ -16,12 +16,11 @@
 //         ops.rs:384-389, applied before the store in forward.rs:300-302).
 //         A layer kept at hi/lo precision also gets the lo halves,
 //         bf16(x - bf16(x)), of K and V in planes laid out like K and V^T.
-//         One launch, one workgroup per (64-row block, 64-wide head-dim
-//         chunk, kv head): K converted in registers, V transposed through LDS.
-//         Rows that fill whole 32-key tiles at contiguous positions, without
-//         RoPE or lo halves (the denoise step's canvas rows), take a second
-//         kernel: one workgroup per (kv head, tile), whole-line loads and
-//         stores.
+//         One launch.  Rows at contiguous positions (canvas, prompt): one
+//         workgroup per (kv head, 32-key tile), whole-line loads and stores.
+//         Position lists and padded head dims: one workgroup per (64-row
+//         block, 64-wide head-dim chunk, kv head), K converted in registers,
+//         V transposed through LDS.
 // gather: StepCache::gather (cache.rs:73-82) -- bf16 back to f32 rows (hi +
 //         lo where the layer keeps the lo halves).
 #include <algorithm>
@@ -378,29 +377,18 @@ __global__ __launch_bounds__(256) void kv_store_kernel(const StoreArgs a) {
 }
 
 // The store of rows that fill whole 32-key V^T tiles at contiguous positions
-// (pos0 and n multiples of 32), head dim == HD (64, 128 or 256), without lo
-// halves: the canvas rows of every denoise step.  One workgroup per (kv
-// head, tile); thread (rg, dc), rg fastest, holds the 4 dims 4 dc .. 4 dc + 3
-// of the tile's rows RPG rg .. RPG rg + RPG - 1.
-// - Loads: per instruction the wave reads whole 128-byte lines (hd 128: 8
-//   rows x 128 B), against 64-byte pieces at a 64-byte lane stride in
-//   kv_store_kernel.
-// - The K / V biases, the K norm and Gemma's V norm of the epilogue, as in
-//   kv_store_kernel: a row's f32 squares summed in f64, over the 4 dims of
-//   each thread, then across the lanes of the row in the wave (shuffles),
-//   then across the 4 waves in wave order (LDS).  RoPE on K (rotate_rows,
-//   ops.rs:433-452; rot a multiple of 8, so a thread's 4 dims lie on one side
-//   of rot / 2) reads the partner dim d +- rot / 2 of the normed row from LDS
-//   and the (sin, cos) pairs of the row's position, loaded with the rows.
+// (pos0 and n multiples of 32) as they are: no epilogue, no lo halves, head
+// dim == HD (64, 128 or 256).  One workgroup per (kv head, tile) for K and V
+// together; thread (rg, dc), rg fastest, holds the 4 dims 4 dc .. 4 dc + 3
+// of the tile's rows RPG rg .. RPG rg + RPG - 1.  With nothing to compute a
+// step's store is a launch and one round trip, and splitting K from V as
+// kv_store_run_kernel does costs more than it gives (C2's 256 rows of 32
+// heads inside a step: 4.9 against 5.2 us).
 // - K: bf16 of the 4 dims, 8 bytes per row.
 // - V^T: at step e the thread writes the RPG keys of its rows in d-row
 //   4 dc + e of the tile; the NRG lanes of one dc together write that
 //   d-row's 64 bytes whole, so no LDS transpose and no barrier is needed.
-// Same values as kv_store_kernel: bf16 (round to nearest even) of each f32.
-// EPI: the epilogue (biases, norms, RoPE) is compiled in; the plain build
-// keeps it out, since its conditional updates of the loaded rows made the K
-// stores wait for every load.
-template <int HD, bool EPI>
+template <int HD>
 __global__ __launch_bounds__(256) void kv_store_tiles_kernel(const StoreArgs a) {
     constexpr int CPR = HD / 4;     // 4-dim pieces per row
     constexpr int NRG = 256 / CPR;  // row groups
@@ -423,104 +411,6 @@ __global__ __launch_bounds__(256) void kv_store_tiles_kernel(const StoreArgs a) 
     for (int j = 0; j < RPG; ++j) {
         xk[j] = *reinterpret_cast<const f32x4*>(a.k + src + j * rstride);
         xv[j] = *reinterpret_cast<const f32x4*>(a.v + src + j * rstride);
-    }
-    if constexpr (EPI) {
-        const int half = a.rot / 2;
-        const int d0 = 4 * dc;
-        const bool rot_me = a.rope && d0 < a.rot;
-        f32x4 tab[RPG][2];  // (sin, cos) of pairs jj .. jj + 3 at each row's position
-        if (rot_me) {
-            const int jj = d0 < half ? d0 : d0 - half;
-            const int pp = (a.pos0 >= 0 ? a.pos0 : 0) + r0;
-#pragma unroll
-            for (int j = 0; j < RPG; ++j) {
-                const float* t = a.rope + ((size_t)(pp + j) * half + jj) * 2;
-                tab[j][0] = *reinterpret_cast<const f32x4*>(t);
-                tab[j][1] = *reinterpret_cast<const f32x4*>(t + 4);
-            }
-        }
-        f32x4 kw4 = {}, kb4 = {}, vb4 = {};
-        if (a.kn_w) kw4 = *reinterpret_cast<const f32x4*>(a.kn_w + 4 * dc);
-        if (a.kb) kb4 = *reinterpret_cast<const f32x4*>(a.kb + (size_t)g * HD + 4 * dc);
-        if (a.vb) vb4 = *reinterpret_cast<const f32x4*>(a.vb + (size_t)g * HD + 4 * dc);
-        // (each bias only where given: adding a zero would turn -0.0 into +0.0)
-        if (a.kb) {
-#pragma unroll
-            for (int j = 0; j < RPG; ++j) xk[j] += kb4;
-        }
-        if (a.vb) {
-#pragma unroll
-            for (int j = 0; j < RPG; ++j) xv[j] += vb4;
-        }
-        if (a.kn_w || a.v_norm) {
-            // rms_norm_inplace (ops.rs:106-114) / rms_norm_noscale: sum of the
-            // row's f32 squares in f64; the row's lanes in this wave are lanes
-            // rg + NRG i, the other CPR / (64 / NRG) - 1 shares are in the
-            // other waves
-            __shared__ double s_ss[2][4][VT_KEYS];  // [K, V][wave][row of the tile]
-            const int wave = tid >> 6;
-            auto row_ss = [&](const f32x4 (&x)[RPG], double (&ss)[RPG]) __attribute__((always_inline)) {
-#pragma unroll
-                for (int j = 0; j < RPG; ++j) {
-                    double t = 0.0;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float sq = x[j][e] * x[j][e];
-                        t += (double)sq;
-                    }
-#pragma unroll
-                    for (int off = NRG; off < 64; off <<= 1) t += __shfl_xor(t, off);
-                    ss[j] = t;
-                }
-            };
-            double ssk[RPG], ssv[RPG];
-            if (a.kn_w) row_ss(xk, ssk);
-            if (a.v_norm) row_ss(xv, ssv);
-            if ((tid & 63) < NRG) {
-#pragma unroll
-                for (int j = 0; j < RPG; ++j) {
-                    if (a.kn_w) s_ss[0][wave][rg * RPG + j] = ssk[j];
-                    if (a.v_norm) s_ss[1][wave][rg * RPG + j] = ssv[j];
-                }
-            }
-            __syncthreads();
-            auto scale_of = [&](int kv, int j) __attribute__((always_inline)) {
-                const double t = ((s_ss[kv][0][rg * RPG + j] + s_ss[kv][1][rg * RPG + j]) + s_ss[kv][2][rg * RPG + j]) +
-                                 s_ss[kv][3][rg * RPG + j];
-                return 1.0f / (float)sqrt(t / (double)HD + (double)a.kn_eps);
-            };
-#pragma unroll
-            for (int j = 0; j < RPG; ++j) {
-                if (a.kn_w) {
-                    const float sc = scale_of(0, j);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) xk[j][e] = xk[j][e] * sc * kw4[e];
-                }
-                if (a.v_norm) {
-                    const float sc = scale_of(1, j);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) xv[j][e] *= sc;
-                }
-            }
-        }
-        if (a.rope) {
-            __shared__ __align__(16) float s_k[VT_KEYS][HD + 4];  // the tile's normed K rows
-#pragma unroll
-            for (int j = 0; j < RPG; ++j) *reinterpret_cast<f32x4*>(&s_k[rg * RPG + j][d0]) = xk[j];
-            __syncthreads();
-            if (rot_me) {
-                const int pd0 = d0 < half ? d0 + half : d0 - half;
-#pragma unroll
-                for (int j = 0; j < RPG; ++j) {
-                    const f32x4 xp = *reinterpret_cast<const f32x4*>(&s_k[rg * RPG + j][pd0]);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float sn = tab[j][e >> 1][2 * (e & 1)], cs = tab[j][e >> 1][2 * (e & 1) + 1];
-                        xk[j][e] = d0 < half ? rope_lo(xk[j][e], xp[e], sn, cs) : rope_hi(xp[e], xk[j][e], sn, cs);
-                    }
-                }
-            }
-        }
     }
     const int p0 = a.pos0 >= 0 ? a.pos0 : 0;  // (host: pos0 >= 0, or no position list)
     uint16_t* kdst = a.kc + ((size_t)g * a.cap + p0 + r0) * HD + 4 * dc;
@@ -549,6 +439,193 @@ __global__ __launch_bounds__(256) void kv_store_tiles_kernel(const StoreArgs a) 
     }
 }
 
+// The store of rows at contiguous positions, head dim == HD: the canvas rows
+// of a denoise step, the prompt, a first pass.  One workgroup per (kv head,
+// 32-key tile that the rows touch, K or V); rows need not fill the first and
+// the last tile.  K and V take a workgroup each, so a step's few tiles give
+// twice the workgroups, each with half the loads to wait for.
+// Thread (rg, dc), rg fastest, holds keys 4 rg .. 4 rg + 3 of the tile at
+// dims 4 dc .. + 3 and HD / 2 + 4 dc .. + 3.
+// - Loads: an instruction reads 8 rows x 128 bytes, whole lines.
+// - K: with a full rotary a dim and its partner d + HD / 2 are in one thread
+//   (a partial rotary takes the partner from LDS).  bf16 of 4 dims, 8 bytes
+//   per row and half.
+// - V^T: the thread writes its 4 keys of a d-row as 8 bytes, so the 8 lanes
+//   of one dc write that d-row's 64 bytes whole, without a transpose in LDS.
+//   A row group that is only partly stored (the ends of the run) writes its
+//   keys one by one.
+// - Norms: f32 squares summed in f64, over the thread's dims, the row's lanes
+//   of the wave (shuffles) and the waves in order (LDS).
+// HBM-bound where it is large, latency-bound in a step.  Against the general
+// kernel (64-row blocks, every thread loading the whole row again for the
+// norms), which took runs that fill no whole tiles, hi/lo layers and head dim
+// 512 before: see the figures at launch_store.
+// EPI: biases, norms and RoPE are compiled in (the plain build keeps them
+// out: its stores then wait for their own loads only).  HILO: the lo planes
+// are written too.
+template <int HD, bool EPI, bool HILO>
+__global__ __launch_bounds__(HD) void kv_store_run_kernel(const StoreArgs a) {
+    constexpr int RPG = 4, NRG = VT_KEYS / RPG;  // rows per thread, row groups
+    constexpr int NWV = HD / 64;                 // waves
+    const int x = blockIdx.x & 7;  // (XCD placement as kv_store_kernel)
+    if (x < a.xcd_lo || x >= a.xcd_lo + a.xcd_n) return;
+    const int lid = (x - a.xcd_lo) * a.per_xcd + (int)(blockIdx.x >> 3);
+    if (lid >= a.n_head_kv * a.n_rb * 2) return;
+    const int g = lid / (2 * a.n_rb), rest = lid - g * 2 * a.n_rb;
+    const bool is_v = rest & 1;
+    const int kt = a.pos0 / VT_KEYS + (rest >> 1);  // key tile
+    const int tid = threadIdx.x, rg = tid % NRG, dc = tid / NRG;
+    const int p0 = kt * VT_KEYS + rg * RPG;  // first position of this thread
+    const int r0 = p0 - a.pos0;              // its row (rows outside [0, n) are not stored)
+    const float* src = (is_v ? a.v : a.k) + (size_t)g * HD + 4 * dc;
+    f32x4 xa[RPG], xb[RPG];  // dims 4 dc .., dims HD / 2 + 4 dc ..
+#pragma unroll
+    for (int j = 0; j < RPG; ++j) {
+        const float* row = src + (size_t)min(max(r0 + j, 0), a.n - 1) * a.rstride;
+        xa[j] = *reinterpret_cast<const f32x4*>(row);
+        xb[j] = *reinterpret_cast<const f32x4*>(row + HD / 2);
+    }
+    if constexpr (EPI) {
+        const int half = a.rot / 2;
+        const bool rope = a.rope && !is_v;
+        // (sin, cos) of pairs jj .. jj + 3 at each row's position, for each
+        // of the thread's two pieces; a full rotary's two pieces share theirs
+        f32x4 ta[RPG][2], tb[RPG][2];
+        const int da = 4 * dc, db = HD / 2 + 4 * dc;
+        auto table = [&](f32x4 (&t)[RPG][2], int d0) __attribute__((always_inline)) {
+            const int jj = d0 < half ? d0 : d0 - half;
+#pragma unroll
+            for (int j = 0; j < RPG; ++j) {
+                const int pos = a.pos0 + min(max(r0 + j, 0), a.n - 1);
+                const float* e = a.rope + ((size_t)pos * half + jj) * 2;
+                t[j][0] = *reinterpret_cast<const f32x4*>(e);
+                t[j][1] = *reinterpret_cast<const f32x4*>(e + 4);
+            }
+        };
+        if (rope && da < a.rot) table(ta, da);
+        if (rope && a.rot != HD && db < a.rot) table(tb, db);
+        const float* bias = is_v ? a.vb : a.kb;
+        const float* gain = is_v ? nullptr : a.kn_w;
+        const bool norm = is_v ? a.v_norm != 0 : a.kn_w != nullptr;
+        f32x4 wa = {}, wb = {};
+        if (gain) {
+            wa = *reinterpret_cast<const f32x4*>(gain + da);
+            wb = *reinterpret_cast<const f32x4*>(gain + db);
+        }
+        if (bias) {  // (only where given: adding a zero would turn -0.0 into +0.0)
+            const f32x4 ba = *reinterpret_cast<const f32x4*>(bias + (size_t)g * HD + da);
+            const f32x4 bb = *reinterpret_cast<const f32x4*>(bias + (size_t)g * HD + db);
+#pragma unroll
+            for (int j = 0; j < RPG; ++j) {
+                xa[j] += ba;
+                xb[j] += bb;
+            }
+        }
+        if (norm) {  // rms_norm_inplace (ops.rs:106-114) / rms_norm_noscale
+            __shared__ double s_ss[NWV][VT_KEYS];
+#pragma unroll
+            for (int j = 0; j < RPG; ++j) {
+                double t = 0.0;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float v = e < 4 ? xa[j][e & 3] : xb[j][e & 3];
+                    const float sq = v * v;
+                    t += (double)sq;
+                }
+#pragma unroll
+                for (int off = NRG; off < 64; off <<= 1) t += __shfl_xor(t, off);
+                if ((tid & 63) < NRG) s_ss[tid >> 6][rg * RPG + j] = t;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < RPG; ++j) {
+                double t = s_ss[0][rg * RPG + j];
+#pragma unroll
+                for (int w = 1; w < NWV; ++w) t += s_ss[w][rg * RPG + j];
+                const float sc = 1.0f / (float)sqrt(t / (double)HD + (double)a.kn_eps);
+                if (gain) {
+                    xa[j] = xa[j] * sc * wa;
+                    xb[j] = xb[j] * sc * wb;
+                } else {
+                    xa[j] *= sc;
+                    xb[j] *= sc;
+                }
+            }
+        }
+        if (rope && a.rot == HD) {
+#pragma unroll
+            for (int j = 0; j < RPG; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float sn = ta[j][e >> 1][2 * (e & 1)], cs = ta[j][e >> 1][2 * (e & 1) + 1];
+                    const float lo = xa[j][e], hi = xb[j][e];
+                    xa[j][e] = rope_lo(lo, hi, sn, cs);
+                    xb[j][e] = rope_hi(lo, hi, sn, cs);
+                }
+        } else if (rope) {
+            if constexpr (HD <= 256) {  // (host: a partial rotary at 512 takes kv_store_kernel)
+                __shared__ __align__(16) float s_k[VT_KEYS][HD + 4];
+#pragma unroll
+                for (int j = 0; j < RPG; ++j) {
+                    *reinterpret_cast<f32x4*>(&s_k[rg * RPG + j][da]) = xa[j];
+                    *reinterpret_cast<f32x4*>(&s_k[rg * RPG + j][db]) = xb[j];
+                }
+                __syncthreads();
+                auto rotate = [&](f32x4 (&y)[RPG], const f32x4 (&t)[RPG][2], int d0) __attribute__((always_inline)) {
+                    const int pd = d0 < half ? d0 + half : d0 - half;
+#pragma unroll
+                    for (int j = 0; j < RPG; ++j) {
+                        const f32x4 yp = *reinterpret_cast<const f32x4*>(&s_k[rg * RPG + j][pd]);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float sn = t[j][e >> 1][2 * (e & 1)], cs = t[j][e >> 1][2 * (e & 1) + 1];
+                            y[j][e] = d0 < half ? rope_lo(y[j][e], yp[e], sn, cs) : rope_hi(yp[e], y[j][e], sn, cs);
+                        }
+                    }
+                };
+                if (da < a.rot) rotate(xa, ta, da);
+                if (db < a.rot) rotate(xb, tb, db);
+            }
+        }
+    }
+    // the bf16 halves: hi, and lo = bf16 of what that rounding dropped
+    auto put = [&](uint16_t* plane, auto conv) __attribute__((always_inline)) {
+        if (!is_v) {
+            uint16_t* dst = plane + ((size_t)g * a.cap + p0) * HD + 4 * dc;
+#pragma unroll
+            for (int j = 0; j < RPG; ++j) {
+                if (r0 + j < 0 || r0 + j >= a.n) continue;
+                *reinterpret_cast<uint2*>(dst + (size_t)j * HD) =
+                    make_uint2((uint32_t)conv(xa[j][0]) | ((uint32_t)conv(xa[j][1]) << 16),
+                               (uint32_t)conv(xa[j][2]) | ((uint32_t)conv(xa[j][3]) << 16));
+                *reinterpret_cast<uint2*>(dst + (size_t)j * HD + HD / 2) =
+                    make_uint2((uint32_t)conv(xb[j][0]) | ((uint32_t)conv(xb[j][1]) << 16),
+                               (uint32_t)conv(xb[j][2]) | ((uint32_t)conv(xb[j][3]) << 16));
+            }
+            return;
+        }
+        uint16_t* dst = plane + (size_t)g * HD * a.cap + (size_t)kt * (HD * VT_KEYS) + rg * RPG;
+        const bool whole = r0 >= 0 && r0 + RPG <= a.n;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            uint16_t* row = dst + (size_t)((e < 4 ? 0 : HD / 2) + 4 * dc + (e & 3)) * VT_KEYS;
+            uint16_t h[RPG];
+#pragma unroll
+            for (int j = 0; j < RPG; ++j) h[j] = conv(e < 4 ? xa[j][e & 3] : xb[j][e & 3]);
+            if (whole) {
+                *reinterpret_cast<uint2*>(row) =
+                    make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+            } else {
+#pragma unroll
+                for (int j = 0; j < RPG; ++j)
+                    if (r0 + j >= 0 && r0 + j < a.n) row[j] = h[j];
+            }
+        }
+    };
+    put(is_v ? a.vtc : a.kc, [](float v) { return f2bf(v); });
+    if constexpr (HILO) put(is_v ? a.vlo : a.klo, [](float v) { return f2bf(v - bf2f(f2bf(v))); });
+}
+
 // One thread per (row, kv head, d).
 template <int HD>
 __global__ __launch_bounds__(256) void kv_gather_kernel(const GatherArgs a) {
@@ -568,6 +645,21 @@ __global__ __launch_bounds__(256) void kv_gather_kernel(const GatherArgs a) {
     }
 }
 
+template <int HD>
+void launch_run(const StoreArgs& a, bool epi, dim3 grid, hipStream_t st) {
+    if (a.klo) {
+        if (epi)
+            hipLaunchKernelGGL((kv_store_run_kernel<HD, true, true>), grid, dim3(HD), 0, st, a);
+        else
+            hipLaunchKernelGGL((kv_store_run_kernel<HD, false, true>), grid, dim3(HD), 0, st, a);
+    } else {
+        if (epi)
+            hipLaunchKernelGGL((kv_store_run_kernel<HD, true, false>), grid, dim3(HD), 0, st, a);
+        else
+            hipLaunchKernelGGL((kv_store_run_kernel<HD, false, false>), grid, dim3(HD), 0, st, a);
+    }
+}
+
 }  // namespace
 
 hipError_t launch_store(int hd_tile, const StoreArgs& args, hipStream_t st) {
@@ -581,24 +673,46 @@ hipError_t launch_store(int hd_tile, const StoreArgs& args, hipStream_t st) {
     const int nb = a.n_batch > 0 ? a.n_batch : 1;
     a.xcd_lo = 8 * a.batch / nb;
     a.xcd_n = std::max(1, 8 * (a.batch + 1) / nb - a.xcd_lo);
-    // whole tiles at contiguous positions, no epilogue: the tile kernel
+    // Rows at contiguous positions whose head dim fills its tile: the tile
+    // kernel where they are whole tiles to be stored as they are, else the
+    // run kernel.  Position lists, padded head dims, rows that are not 16-byte
+    // aligned and a partial rotary at head dim 512 take the general kernel.
+    // Run kernel against the kernels that took these calls before (general;
+    // * the tile kernel with an epilogue), in us, kernel times:
+    //   16 heads, hd 128, 512 rows from position 2041, norm + RoPE   12.5 / 7.0
+    //   8 heads, hd 256, 256 rows, hi/lo, norms + RoPE               11.9 / 7.7
+    //   2 heads, hd 512, 256 rows, hi/lo, norms + RoPE               20.7 / 12.3
+    //   8 heads, hd 256, 4352 rows, hi/lo, norms + RoPE               121 / 47.7
+    //   4 heads, hd 128, 1280 rows, bias + RoPE *                     7.8 / 6.5
+    //   32 heads, hd 128, 64 rows, RoPE *                             5.1 / 4.0
     const int p0 = a.pos0 >= 0 ? a.pos0 : (a.pos == nullptr ? 0 : -1);
-    const bool tiles = a.vec && a.hd == hd_tile && hd_tile <= 256 && p0 >= 0 && p0 % VT_KEYS == 0 &&
-                       a.n % VT_KEYS == 0 && !a.klo && !a.vlo && (!a.rope || (a.rot % 8 == 0 && a.rot <= a.hd)) &&
-                       (((uintptr_t)a.kn_w | (uintptr_t)a.kb | (uintptr_t)a.vb | (uintptr_t)a.rope) & 15) == 0;
-    if (tiles) {
+    const bool rot_ok = !a.rope || a.rot == a.hd || (hd_tile <= 256 && a.rot % 8 == 0 && a.rot <= a.hd);
+    const bool run = a.vec && a.hd == hd_tile && p0 >= 0 && rot_ok && !a.klo == !a.vlo &&
+                     (((uintptr_t)a.kn_w | (uintptr_t)a.kb | (uintptr_t)a.vb | (uintptr_t)a.rope) & 15) == 0;
+    const bool epi = a.kn_w || a.kb || a.vb || a.v_norm || a.rope;
+    if (run && !epi && !a.klo && hd_tile <= 256 && p0 % VT_KEYS == 0 && a.n % VT_KEYS == 0) {
         a.pos0 = p0;
         const int work = a.n_head_kv * (a.n / VT_KEYS);
         a.per_xcd = (work + a.xcd_n - 1) / a.xcd_n;
         const dim3 grid((unsigned)(8 * a.per_xcd));
-        const bool epi = a.kn_w || a.kb || a.vb || a.v_norm || a.rope;
-        switch (hd_tile * 2 + (epi ? 1 : 0)) {
-            case 128: hipLaunchKernelGGL((kv_store_tiles_kernel<64, false>), grid, dim3(256), 0, st, a); break;
-            case 129: hipLaunchKernelGGL((kv_store_tiles_kernel<64, true>), grid, dim3(256), 0, st, a); break;
-            case 256: hipLaunchKernelGGL((kv_store_tiles_kernel<128, false>), grid, dim3(256), 0, st, a); break;
-            case 257: hipLaunchKernelGGL((kv_store_tiles_kernel<128, true>), grid, dim3(256), 0, st, a); break;
-            case 512: hipLaunchKernelGGL((kv_store_tiles_kernel<256, false>), grid, dim3(256), 0, st, a); break;
-            default: hipLaunchKernelGGL((kv_store_tiles_kernel<256, true>), grid, dim3(256), 0, st, a); break;
+        switch (hd_tile) {
+            case 64: hipLaunchKernelGGL(kv_store_tiles_kernel<64>, grid, dim3(256), 0, st, a); break;
+            case 128: hipLaunchKernelGGL(kv_store_tiles_kernel<128>, grid, dim3(256), 0, st, a); break;
+            default: hipLaunchKernelGGL(kv_store_tiles_kernel<256>, grid, dim3(256), 0, st, a); break;
+        }
+        return hipGetLastError();
+    }
+    if (run) {
+        a.pos0 = p0;
+        a.n_rb = (p0 + a.n - 1) / VT_KEYS - p0 / VT_KEYS + 1;
+        const int work = a.n_head_kv * a.n_rb * 2;
+        a.per_xcd = (work + a.xcd_n - 1) / a.xcd_n;
+        const dim3 grid((unsigned)(8 * a.per_xcd));
+        switch (hd_tile) {
+            case 64: launch_run<64>(a, epi, grid, st); break;
+            case 128: launch_run<128>(a, epi, grid, st); break;
+            case 256: launch_run<256>(a, epi, grid, st); break;
+            default: launch_run<512>(a, epi, grid, st); break;
         }
         return hipGetLastError();
     }
