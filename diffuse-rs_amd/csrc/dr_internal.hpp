@@ -171,7 +171,8 @@ struct Q8KBlock {
 static_assert(sizeof(Q8KBlock) == 292, "Q8_K block layout");
 
 // Activation rows of dr_qmatmul's workspace: a multiple of the 128 rows of a
-// qmm workgroup (the pad rows are quantized as zeros).
+// qmm workgroup (the pad rows are quantized as zeros).  The slice kernels
+// read whole 32-row tiles up to 64 rows at a time.
 __host__ __device__ inline int qmm_rows_padded(int n) { return (n + 127) / 128 * 128; }
 
 // dr_qmatmul's workspace: the Q8_K activations in the order the int8 MFMA

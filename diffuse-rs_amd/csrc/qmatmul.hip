@@ -237,6 +237,7 @@ __global__ __launch_bounds__(512) void q8k_quantize_tiles_kernel(const float* __
 // slab s of row c; accumulator slot i of that lane is output (t = 8 (i / 4) +
 // 4 g + i % 4, r = c).
 //
+// (This kernel runs Q4_K only; Q6_K always takes qmm_slice_kernel below.)
 // Weight operand of a Q4_K block: slab s = sub-block s.  sc_s = 8 sh + sl with
 // sh, sl <= 7, so sh * q and sl * q (q <= 15) are bytes and a 16-bit packed
 // multiply scales two nibble bytes at once without carries; the two parts
@@ -287,9 +288,9 @@ struct BlockScale {
     bf16x8 mn;  // Q4_K: the eight 6-bit mins (B operand of the min MFMA)
 };
 
-// Scales of a block, and this wave's two slabs of B operands into LDS
-// (dst[slab][hi / lo][lane]).
-__device__ __forceinline__ void prep(const RawBlock<12>& r, int c, int lane, u32x4* dst, BlockScale& o) {
+// Scales of a block, and the B operands of its slabs 2 c and 2 c + 1 (w[slab][hi
+// / lo]); prep writes them to LDS (dst[slab][hi / lo][lane]).
+__device__ __forceinline__ void form_pair(const RawBlock<12>& r, int c, int lane, u32x4 (&w)[2][2], BlockScale& o) {
     const u32x4 h = r.h;
     o.wd = f16_to_f32(h.x & 0xFFFF);
     o.wdmin = f16_to_f32(h.x >> 16);
@@ -315,12 +316,12 @@ __device__ __forceinline__ void prep(const RawBlock<12>& r, int c, int lane, u32
             vh[k] = pk_mul_u16(nib, fh);
             vl[k] = pk_mul_u16(nib, fl);
         }
-        dst[((2 * c + hn) * 2 + 0) * 64 + lane] = vh;
-        dst[((2 * c + hn) * 2 + 1) * 64 + lane] = vl;
+        w[hn][0] = vh;
+        w[hn][1] = vl;
     }
 }
 
-__device__ __forceinline__ void prep(const RawBlock<14>& r, int c, int lane, u32x4* dst, BlockScale& o) {
+__device__ __forceinline__ void form_pair(const RawBlock<14>& r, int c, int lane, u32x4 (&w)[2][2], BlockScale& o) {
     o.wd = f16_to_f32(r.d);
     o.wdmin = 0.0f;
     const int g = lane >> 5;
@@ -345,9 +346,19 @@ __device__ __forceinline__ void prep(const RawBlock<14>& r, int c, int lane, u32
             vh[k] = pack_lo_bytes(pk_ashr_i16(w01, 6), pk_ashr_i16(w23, 6));
             vl[k] = pack_lo_bytes(w01 & 0x003F003Fu, w23 & 0x003F003Fu);
         }
-        dst[(s * 2 + 0) * 64 + lane] = vh;
-        dst[(s * 2 + 1) * 64 + lane] = vl;
+        w[k2][0] = vh;
+        w[k2][1] = vl;
     }
+}
+
+template <int WT>
+__device__ __forceinline__ void prep(const RawBlock<WT>& r, int c, int lane, u32x4* dst, BlockScale& o) {
+    u32x4 w[2][2];
+    form_pair(r, c, lane, w, o);
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) dst[((2 * c + s) * 2 + p) * 64 + lane] = w[s][p];
 }
 
 // The residual of a lane's 16 outputs (activation rows t0 + 8 (i / 4) + 4 g
@@ -377,11 +388,9 @@ __device__ __forceinline__ void store_tile(const QmmArgs& a, int t0, int g, int 
     }
 }
 
-template <int WT>
 __global__ __launch_bounds__(512) void qmm_kernel(const QmmArgs a) {
-    constexpr bool Q4 = WT == 12;
-    constexpr int WB = Q4 ? Q4K_BYTES : Q6K_BYTES;
-    constexpr int SHIFT = Q4 ? 3 : 6;
+    constexpr int WB = Q4K_BYTES;
+    constexpr int SHIFT = 3;
     // B operands [buffer][half][slab][hi / lo][lane] (64 KB); after the loop
     // the first 16 KB carry half 1's partial sums [tile][slot][lane]
     __shared__ u32x4 s_b[2][2][8][2][64];
@@ -424,7 +433,7 @@ __global__ __launch_bounds__(512) void qmm_kernel(const QmmArgs a) {
         bf16x8 bm;
     };
     Stage S[2];
-    RawBlock<WT> R[2];
+    RawBlock<12> R[2];
     BlockScale bsc;
     const int blast = kb0 + (kcnt > 0 ? kcnt - 1 : 0);
     auto load_stage = [&](int b, Stage& st) __attribute__((always_inline)) {
@@ -432,7 +441,7 @@ __global__ __launch_bounds__(512) void qmm_kernel(const QmmArgs a) {
 #pragma unroll
         for (int s = 0; s < 8; ++s) st.av[s] = gld<i32x4>(abase + ((size_t)b * 8 + s) * 1024);
         st.xd = gld<float>(xbase + (size_t)b * 32);
-        if constexpr (Q4) st.bm = gld<bf16x8>(mbase + (size_t)b * 64 * 8);
+        st.bm = gld<bf16x8>(mbase + (size_t)b * 64 * 8);
     };
     // The combine of a block runs in the next iteration, under that block's
     // MFMA chains: the products of the previous block wait in registers.
@@ -446,10 +455,10 @@ __global__ __launch_bounds__(512) void qmm_kernel(const QmmArgs a) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             sum[i] = __builtin_fmaf(pr.dd[i], (float)pr.acc[i], sum[i]);
-            if constexpr (Q4) sum[i] = __builtin_fmaf(-pr.dm[i], pr.mins[i], sum[i]);
+            sum[i] = __builtin_fmaf(-pr.dm[i], pr.mins[i], sum[i]);
         }
     };
-    auto body = [&](int it, Stage& cur, Stage& nxt, RawBlock<WT>& rprep, RawBlock<WT>& rload, int buf)
+    auto body = [&](int it, Stage& cur, Stage& nxt, RawBlock<12>& rprep, RawBlock<12>& rload, int buf)
         __attribute__((always_inline)) {
         if (it < kcnt) {
             load_stage(min(kb0 + it + 1, blast), nxt);
@@ -474,14 +483,14 @@ __global__ __launch_bounds__(512) void qmm_kernel(const QmmArgs a) {
                     cur.av[s], __builtin_bit_cast(i32x4, bsrc[(s * 2 + 1) * 64]), acc, 0, 0, 0);
             np.acc = acc;
             np.mins = f32x16{};
-            if constexpr (Q4) np.mins = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.bm, bsc.mn, np.mins, 0, 0, 0);
+            np.mins = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.bm, bsc.mn, np.mins, 0, 0, 0);
             // the block scales d_x d_w (and d_x dmin_w) of every slot, each one
             // f32 product, on a K = 2 f32 MFMA with the second K row zero
             const float xa = g == 0 ? cur.xd : 0.0f;
             const f32x16 z = {};
             np.dd = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, g == 0 ? bsc.wd : 0.0f, z, 0, 0, 0);
             np.dm = f32x16{};
-            if constexpr (Q4) np.dm = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, g == 0 ? bsc.wdmin : 0.0f, z, 0, 0, 0);
+            np.dm = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, g == 0 ? bsc.wdmin : 0.0f, z, 0, 0, 0);
             // ---- under the second chain: the next block's B operands into the
             // other buffer (past the last block: a repeat nobody reads)
             prep(rprep, c, lane, &s_b[buf ^ 1][kh][0][0][0], bsc);
@@ -491,7 +500,7 @@ __global__ __launch_bounds__(512) void qmm_kernel(const QmmArgs a) {
         lds_barrier();
     };
     if (kcnt > 0) {
-        RawBlock<WT> raw0;
+        RawBlock<12> raw0;
         load_raw(wrow + (size_t)kb0 * WB, c, g, raw0);
         load_stage(kb0, S[0]);
         load_raw(wrow + (size_t)min(kb0 + 1, blast) * WB, c, g, R[1]);
@@ -782,6 +791,275 @@ __global__ __launch_bounds__(512) void qmm0_kernel(const QmmArgs a) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// Slices of the blocks: calls whose grid would leave CUs idle (an MoE
+// expert's rows, short canvases), and all of Q6_K; see use_slices.  The
+// kernels that walk every block take one memory round trip after the other
+// (a block or a group of blocks, then a barrier).  Here the 8 waves of a
+// workgroup take an eighth of the blocks each, for 32 weight rows and TT tiles
+// of 32 activation rows: a wave forms its own weight operands (no wave
+// shares them, so the loop has no barrier), keeps several blocks' loads in
+// flight and uses each operand for TT tiles.  The eighths meet in LDS and are
+// added in their order, so every output is summed in one fixed order.
+// 1024 x 2048 Q8_0 weights, up to 32 rows, kernel alone: 14.2 -> 6.1 us; 64
+// rows 8.4.
+template <int TT>
+__device__ __forceinline__ void finish_slices(const QmmArgs& a, const f32x16 (&sum)[TT], float (&s_red)[8][16][64],
+                                              int wave, int lane, int t0, int rt) {
+    const int c = lane & 31, g = lane >> 5;
+    const int rr = rt * 32 + c;
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+        if (tt > 0) lds_barrier();  // the tile before is read
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s_red[wave][i][lane] = sum[tt][i];
+        lds_barrier();
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int i = wave + 8 * k;
+            const int t = t0 + 32 * tt + 8 * (i >> 2) + 4 * g + (i & 3);
+            float v = s_red[0][i][lane];
+#pragma unroll
+            for (int w = 1; w < 8; ++w) v = v + s_red[w][i][lane];
+            if (t < a.n && rr < a.rows) {
+                if (a.residual) v += gld<float>(a.residual + (size_t)t * a.rows + rr);
+                a.out[(size_t)t * a.rows + rr] = v;
+            }
+        }
+    }
+}
+
+// The 32-value block types.  Lane (c, g): weight row c, activation row c of
+// each tile, values 16 g .. + 15 of a block (as qmm0_kernel).
+//
+// A block is 18, 22 or 34 bytes, so a lane's 16 bytes of its row lie at any
+// even address: loaded directly, each instruction touches 32 rows and two
+// lines in many of them, and the address unit set the pace (1024 x 2048
+// Q8_0, 32 rows: 13.5 us).  So a wave reads CB blocks of its 32 rows as
+// 16-byte pieces in row order, from a 4-byte boundary on, through a buffer
+// resource that ends with the weights (pieces past them read as zeros), puts
+// them into its own part of LDS and shifts its bytes out of dwords there.
+template <int WT>
+struct SliceGeom {
+    static constexpr int BB = WT == 2 ? 18 : (WT == 6 ? 22 : 34);
+    static constexpr int CB = WT == 8 ? 4 : 8;            // blocks per chunk
+    static constexpr int NP = (CB * BB + 2 + 15) / 16;    // 16-byte pieces of a row's chunk (2: the misalignment)
+    static constexpr int NL = (32 * NP + 63) / 64;        // loads per lane
+    static constexpr int RS = (NP * 4) | 1;               // dwords per row in LDS (odd: rows on distinct banks)
+};
+template <int WT, int TT>
+__global__ __launch_bounds__(512) void qmm0_slice_kernel(const QmmArgs a) {
+    using G = SliceGeom<WT>;
+    constexpr int BB = G::BB, CB = G::CB, NP = G::NP, NL = G::NL, RS = G::RS;
+    constexpr size_t W_BYTES = sizeof(uint32_t) * 8 * 32 * RS, R_BYTES = sizeof(float) * 8 * 16 * 64;
+    __shared__ __align__(16) char s_mem[W_BYTES > R_BYTES ? W_BYTES : R_BYTES];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 31, g = lane >> 5;
+    const int nb = a.cols / 32;
+    const int n_rt = (a.rows + 31) / 32, tg = blockIdx.x / n_rt, rt = blockIdx.x - tg * n_rt;
+    const int t32 = tg * TT;  // first activation tile
+    const Q0Layout L(a.ws, a.n_pad, a.cols);
+    uint32_t* const sw = reinterpret_cast<uint32_t*>(s_mem) + wave * 32 * RS;
+    const int per = (nb + 7) / 8;
+    const int b0 = min(wave * per, nb), cnt = min(b0 + per, nb) - b0;
+    const int blast = cnt > 0 ? b0 + cnt - 1 : nb - 1;  // (activations past the slice: its last block again)
+
+    // the 32 weight rows, from the 4-byte boundary at or before the first
+    const uint8_t* w0 = static_cast<const uint8_t*>(a.w) + (size_t)rt * 32 * nb * BB;
+    const int mis0 = (int)((uintptr_t)w0 & 3);
+    const int row_b = nb * BB;
+    const int bytes = (mis0 + min(32, a.rows - rt * 32) * row_b + 3) & ~3;
+    const __amdgpu_buffer_rsrc_t rw =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w0 - mis0), 0, bytes, 0x00020000);
+    u32x4 pc[NL];
+    auto load_w = [&](int j) __attribute__((always_inline)) {  // blocks j .. j + CB - 1 of the slice
+#pragma unroll
+        for (int k = 0; k < NL; ++k) {
+            const int idx = k * 64 + lane, row = idx / NP, p = idx - row * NP;
+            const int off = (mis0 + row * row_b + (b0 + j) * BB) & ~3;
+            // (rows past the tile and chunks past the slice: nothing is read)
+            pc[k] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                  rw, row < 32 && j < cnt ? off + 16 * p : bytes, 0, 0));
+        }
+    };
+    auto store_w = [&]() __attribute__((always_inline)) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();  // (the chunk before is read: LDS runs a wave's accesses in order)
+#pragma unroll
+        for (int k = 0; k < NL; ++k) {
+            const int idx = k * 64 + lane, row = idx / NP, p = idx - row * NP;
+            if (row < 32) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sw[row * RS + 4 * p + e] = pc[k][e];
+            }
+        }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+    };
+    struct Act {
+        i32x4 av[TT];
+        float xd[TT];
+    };
+    Act S[CB];
+    auto load_a = [&](int j, Act& st) __attribute__((always_inline)) {
+        const int b = min(b0 + j, blast);
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) {
+            st.av[tt] = gld<i32x4>(L.qs + (((size_t)(t32 + tt) * nb + b) * 64 + lane) * 16);
+            st.xd[tt] = gld<float>(L.xd + ((size_t)(t32 + tt) * nb + b) * 32 + c);
+        }
+    };
+    f32x16 sum[TT];
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sum[tt][i] = 0.0f;
+    const f32x16 z = {};
+    load_w(0);
+#pragma unroll
+    for (int j = 0; j < CB; ++j) load_a(j, S[j]);
+    for (int it = 0; it < cnt; it += CB) {
+        store_w();
+        load_w(it + CB);
+        // this lane's row of the chunk starts mis bytes into its LDS row
+        const int mis = (mis0 + c * row_b + (b0 + it) * BB) & 3;
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            if (it + j < cnt) {
+                LegacyRaw<WT> raw;
+                const uint32_t* row = sw + c * RS;
+                auto at = [&](int byte) __attribute__((always_inline)) {  // 4 bytes at an even offset
+                    const int o = mis + byte;
+                    return __builtin_amdgcn_alignbit(row[(o >> 2) + 1], row[o >> 2], (o & 2) * 8);
+                };
+                const int o = j * BB;
+                raw.dh = at(o) & 0xFFFFu;
+                raw.qh = WT == 6 ? at(o + 2) : 0;
+                const int q = o + (WT == 8 ? 2 + 16 * g : (WT == 2 ? 2 : 6));
+#pragma unroll
+                for (int k = 0; k < 4; ++k) raw.q[k] = at(q + 4 * k);
+                const i32x4 bv = legacy_operand<WT>(raw, g);
+                const float wd = g == 0 ? f16_to_f32(raw.dh) : 0.0f;
+#pragma unroll
+                for (int tt = 0; tt < TT; ++tt) {
+                    const i32x16 acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(S[j].av[tt], bv, i32x16{}, 0, 0, 0);
+                    const f32x16 dd =
+                        __builtin_amdgcn_mfma_f32_32x32x2f32(g == 0 ? S[j].xd[tt] : 0.0f, wd, z, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) sum[tt][i] = __builtin_fmaf((float)acc[i], dd[i], sum[tt][i]);
+                }
+            }
+            load_a(it + CB + j, S[j]);
+        }
+    }
+    __syncthreads();  // the chunks' LDS becomes the slices' sums
+    finish_slices<TT>(a, sum, *reinterpret_cast<float(*)[8][16][64]>(s_mem), wave, lane, t32 * 32, rt);
+}
+
+// The k-quants.  A wave forms the weight operands of its block two slabs at a
+// time (prep of the kernel above, into registers) and multiplies them with
+// every tile; the hi and lo parts run as two accumulators.
+template <int WT, int TT>
+__global__ __launch_bounds__(512) void qmm_slice_kernel(const QmmArgs a) {
+    constexpr bool Q4 = WT == 12;
+    constexpr int WB = Q4 ? Q4K_BYTES : Q6K_BYTES;
+    constexpr int SHIFT = Q4 ? 3 : 6;
+    __shared__ float s_red[8][16][64];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 31, g = lane >> 5;
+    const int nb = a.cols / QK;
+    const int n_rt = (a.rows + 31) / 32, tg = blockIdx.x / n_rt, rt = blockIdx.x - tg * n_rt;
+    const int t32 = tg * TT;  // first activation tile
+    const int r = min(rt * 32 + c, a.rows - 1);
+    const QmmLayout L(a.ws, a.n_pad, a.cols);
+    const uint8_t* wrow = static_cast<const uint8_t*>(a.w) + (size_t)r * nb * WB;
+    const int per = (nb + 7) / 8;
+    const int b0 = min(wave * per, nb), cnt = min(b0 + per, nb) - b0;
+    const int blast = cnt > 0 ? b0 + cnt - 1 : nb - 1;
+    struct Stage {
+        RawBlock<WT> raw[4];  // slabs 2 k, 2 k + 1 (what they share is loaded once: the compiler sees equal addresses)
+        i32x4 av[TT][8];
+        float xd[TT];
+        bf16x8 bm[TT];
+    };
+    auto load = [&](int j, Stage& st) __attribute__((always_inline)) {
+        const int b = min(b0 + j, blast);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) load_raw(wrow + (size_t)b * WB, k, g, st.raw[k]);
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) {
+#pragma unroll
+            for (int s = 0; s < 8; ++s)
+                st.av[tt][s] = gld<i32x4>(L.qs + (((size_t)(t32 + tt) * nb + b) * 8 + s) * 1024 + lane * 16);
+            st.xd[tt] = gld<float>(L.xd + ((size_t)(t32 + tt) * nb + b) * 32 + c);
+            if constexpr (Q4) st.bm[tt] = gld<bf16x8>(L.bmin + (((size_t)(t32 + tt) * nb + b) * 64 + lane) * 8);
+        }
+    };
+    f32x16 sum[TT];
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sum[tt][i] = 0.0f;
+    const f32x16 z = {};
+    // One tile: the next block's loads are in flight under this block.  Two
+    // tiles have no registers for that (a second set of operands spills); a
+    // wave has one or two blocks there, and the other wave of its SIMD runs.
+    constexpr bool AHEAD = TT == 1;
+    Stage S[AHEAD ? 2 : 1];
+    if constexpr (AHEAD) load(0, S[0]);
+    auto block = [&](int it, Stage& cur, Stage& nxt) __attribute__((always_inline)) {
+        load(AHEAD ? it + 1 : it, nxt);
+        __builtin_amdgcn_sched_barrier(0);  // (the loads would sink to their use)
+        BlockScale bsc;
+        i32x16 hi[TT], lo[TT];
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) hi[tt] = lo[tt] = i32x16{};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            u32x4 w[2][2];  // [slab of the pair][hi / lo]
+            form_pair(cur.raw[k], k, lane, w, bsc);
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int tt = 0; tt < TT; ++tt) {
+                    hi[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur.av[tt][2 * k + s],
+                                                                   __builtin_bit_cast(i32x4, w[s][0]), hi[tt], 0, 0, 0);
+                    lo[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur.av[tt][2 * k + s],
+                                                                   __builtin_bit_cast(i32x4, w[s][1]), lo[tt], 0, 0, 0);
+                }
+        }
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) {
+            const float xa = g == 0 ? cur.xd[tt] : 0.0f;
+            const f32x16 dd = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, g == 0 ? bsc.wd : 0.0f, z, 0, 0, 0);
+            f32x16 mins = {}, dm = {};
+            if constexpr (Q4) {
+                mins = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.bm[tt], bsc.mn, mins, 0, 0, 0);
+                dm = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, g == 0 ? bsc.wdmin : 0.0f, z, 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int v = (hi[tt][i] << SHIFT) + lo[tt][i];
+                sum[tt][i] = __builtin_fmaf(dd[i], (float)v, sum[tt][i]);
+                if constexpr (Q4) sum[tt][i] = __builtin_fmaf(-dm[i], mins[i], sum[tt][i]);
+            }
+        }
+    };
+    if constexpr (AHEAD) {
+        int it = 0;
+        for (; it + 1 < cnt; it += 2) {
+            block(it, S[0], S[1]);
+            block(it + 1, S[1], S[0]);
+        }
+        if (it < cnt) block(it, S[0], S[1]);
+    } else {
+        for (int it = 0; it < cnt; ++it) block(it, S[0], S[0]);
+    }
+    finish_slices<TT>(a, sum, s_red, wave, lane, t32 * 32, rt);
+}
+
 // Gemma's post-attention RMSNorm before the residual add (forward.rs:346-350):
 // row t of x ([n][e], the matmul's output) becomes out = x * scale * w +
 // residual, scale = 1 / (float)sqrt(ss / e + eps) with ss the f64 sum of the
@@ -885,6 +1163,44 @@ size_t qmm0_workspace_bytes(int n, int cols) {
     return n_pad * cols + n_pad * nb * sizeof(float);
 }
 
+// The slice kernels (an eighth of the blocks per wave, 32 weight rows x 32 or
+// 64 activation rows per workgroup) or the ones that walk all blocks of 32 x
+// 128.  A walk costs a round trip per block or group of blocks whatever the
+// size, so slices win while their workgroups fit the CUs once; past that the
+// work they repeat per 64 activation rows counts (forming the weight
+// operands, for the 32-value types shifting them out of LDS).  Calls, us,
+// walk / slices, 4096 x 4096 unless noted:
+//   Q4_K  n 20 20.4 / 12.0, 60 21.0 / 15.2, 120 21.2 / 15.9, 190 22.2 / 25.1,
+//         256 22.6 / 25.9; 2048 x 2048 n 256 14.8 / 11.4, 512 16.4 / 18.4
+//   Q4_0  n 20 28.5 / 12.1, 60 29.0 / 17.4, 120 29.3 / 18.3, 256 30.3 / 32.1
+// Q6_K always takes slices: its operands cost more to form than to share
+// through LDS (n 60 34.5 / 17.3, 256 35.7 / 30.9; 2048 x 4096, 2553 rows with
+// the norm, 176 / 134).
+static bool use_slices(const QmmArgs& a) {
+    return a.wtype == 14 || (a.rows + 31) / 32 * ((a.n + 63) / 64) <= 256;
+}
+// Activation tiles that the matmul reads.
+static int quantized_tiles(const QmmArgs& a) {
+    return !use_slices(a) ? a.n_pad / 32 : (a.n <= 32 ? 1 : (a.n + 63) / 64 * 2);
+}
+template <int WT>
+static void launch_slices(const QmmArgs& a, hipStream_t st) {
+    const unsigned n_rt = (unsigned)((a.rows + 31) / 32);
+    const bool one = a.n <= 32;
+    const dim3 grid(n_rt * (one ? 1u : (unsigned)((a.n + 63) / 64)));
+    if constexpr (WT == 12 || WT == 14) {
+        if (one)
+            hipLaunchKernelGGL((qmm_slice_kernel<WT, 1>), grid, dim3(512), 0, st, a);
+        else
+            hipLaunchKernelGGL((qmm_slice_kernel<WT, 2>), grid, dim3(512), 0, st, a);
+    } else {
+        if (one)
+            hipLaunchKernelGGL((qmm0_slice_kernel<WT, 1>), grid, dim3(512), 0, st, a);
+        else
+            hipLaunchKernelGGL((qmm0_slice_kernel<WT, 2>), grid, dim3(512), 0, st, a);
+    }
+}
+
 static bool legacy_wtype(int wt) { return wt == 2 || wt == 6 || wt == 8; }
 
 hipError_t launch_qmatmul(const QmmArgs& a, hipStream_t st) {
@@ -892,7 +1208,7 @@ hipError_t launch_qmatmul(const QmmArgs& a, hipStream_t st) {
     if (legacy_wtype(a.wtype)) {
         if (a.n_pad != qmm_rows_padded(a.n) || a.cols % 32 != 0) return hipErrorInvalidValue;
         const int nb = a.cols / 32;
-        const unsigned items = (unsigned)(a.n_pad / 32 * nb);
+        const unsigned items = (unsigned)(quantized_tiles(a) * nb);
         hipLaunchKernelGGL(q80_quantize_kernel<false>, dim3((items + 3) / 4), dim3(256), 0, st, a.act, a.cols, nb,
                            a.n, a.n_pad, a.ws);
         hipError_t e = hipGetLastError();
@@ -903,10 +1219,18 @@ hipError_t launch_qmatmul(const QmmArgs& a, hipStream_t st) {
             b.residual = nullptr;
             b.out = a.norm_tmp;
         }
-        switch (a.wtype) {
-            case 2: hipLaunchKernelGGL(qmm0_kernel<2>, dim3(nwg), dim3(512), 0, st, b); break;
-            case 6: hipLaunchKernelGGL(qmm0_kernel<6>, dim3(nwg), dim3(512), 0, st, b); break;
-            default: hipLaunchKernelGGL(qmm0_kernel<8>, dim3(nwg), dim3(512), 0, st, b); break;
+        if (use_slices(a)) {
+            switch (a.wtype) {
+                case 2: launch_slices<2>(b, st); break;
+                case 6: launch_slices<6>(b, st); break;
+                default: launch_slices<8>(b, st); break;
+            }
+        } else {
+            switch (a.wtype) {
+                case 2: hipLaunchKernelGGL(qmm0_kernel<2>, dim3(nwg), dim3(512), 0, st, b); break;
+                case 6: hipLaunchKernelGGL(qmm0_kernel<6>, dim3(nwg), dim3(512), 0, st, b); break;
+                default: hipLaunchKernelGGL(qmm0_kernel<8>, dim3(nwg), dim3(512), 0, st, b); break;
+            }
         }
         e = hipGetLastError();
         if (e != hipSuccess || !a.norm_w) return e;
@@ -916,7 +1240,7 @@ hipError_t launch_qmatmul(const QmmArgs& a, hipStream_t st) {
     }
     if (a.n_pad != qmm_rows_padded(a.n) || a.cols % QK != 0) return hipErrorInvalidValue;
     const int nb = a.cols / QK;
-    hipLaunchKernelGGL(q8k_quantize_tiles_kernel, dim3((unsigned)(a.n_pad / 32 * nb)), dim3(512), 0, st, a.act,
+    hipLaunchKernelGGL(q8k_quantize_tiles_kernel, dim3((unsigned)(quantized_tiles(a) * nb)), dim3(512), 0, st, a.act,
                        a.cols, nb, a.n, a.n_pad, a.ws);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -926,12 +1250,13 @@ hipError_t launch_qmatmul(const QmmArgs& a, hipStream_t st) {
         b.residual = nullptr;
         b.out = a.norm_tmp;
     }
-    if (a.wtype == 12)
-        hipLaunchKernelGGL(qmm_kernel<12>, dim3(nwg), dim3(512), 0, st, b);
-    else if (a.wtype == 14)
-        hipLaunchKernelGGL(qmm_kernel<14>, dim3(nwg), dim3(512), 0, st, b);
+    if (a.wtype != 12 && a.wtype != 14) return hipErrorInvalidValue;
+    if (a.wtype == 14)
+        launch_slices<14>(b, st);
+    else if (use_slices(a))
+        launch_slices<12>(b, st);
     else
-        return hipErrorInvalidValue;
+        hipLaunchKernelGGL(qmm_kernel, dim3(nwg), dim3(512), 0, st, b);
     e = hipGetLastError();
     if (e != hipSuccess || !a.norm_w) return e;
     hipLaunchKernelGGL(post_norm_kernel, dim3((unsigned)a.n), dim3(256), 0, st, a.norm_tmp, a.out, a.norm_w,
