@@ -1609,6 +1609,33 @@ LaunchPlan plan_attention(int hd, int n_batch, int n_head_kv, int group, int max
         p.rotate = heads * (long long)(band < max_nk ? band : max_nk) * hd * 4 <= (3LL << 20);
         return p;
     }
+    // Many query rows at head dims 64 and 128: attn_rows_kernel, once its
+    // 64-row workgroups outnumber the CUs (two share one).  Calls with their
+    // store, us, staged / rows (workgroups): Dream 2 x 1280 first pass 107 / 92
+    // (1120), 4 x 256 of 1280 54.3 / 49.9 (448); 32 heads 2560 first pass 193
+    // / 163 (1280), 768 first pass 40.6 / 36.2 (384), 4 x 256 of 768 88 / 82
+    // (512); 8/2 heads of 64, 2 x 4000 first pass 132 / 100 (1000).  At or
+    // below one per CU the staged kernel's 8 waves win: 16 heads 1000 first
+    // pass 30.9 / 31.3 (256), 2 x 256 of 768 32.3 / 33.2 (256), 8/2 heads of
+    // 64 2000 first pass 24.4 / 26.0 (250), Dream 2 x 256 of 1280 28.9 / 31.6
+    // (224).  Workgroups of 128 rows (half the K/V stream) lose to their
+    // longer tail: 92 -> 110, 163 -> 180 in the first two.
+    const int rows_wg = n_batch * n_head_kv * ((row_blocks + 1) / 2);
+    if ((hd == 64 || hd == 128) && mask != MASK_KEYS && (qepi != QEPI_FULL || rot == 0 || rot == hd) &&
+        force_kernel == KERNEL_AUTO && force_rb <= 0 && force_kq <= 0 && force_split <= 0 && force_rows <= 0 &&
+        rows_wg > cus) {
+        p.rows = true;
+        p.rb = 2;
+        p.kq = 2;
+        p.w16 = false;
+        p.qepi = false;  // the Q bias, norm and RoPE are runtime operands of the kernel
+        p.waves = p.rb * p.kq;
+        p.stages = 2;
+        p.rowgroups = (row_blocks + 1) / 2;
+        p.n_split = 1;
+        p.n_workgroups = rows_wg;
+        return p;
+    }
     // Head dims up to 128: one row block of four key groups with four DMA
     // waves (two waves per SIMD).  256: two row blocks of two key groups,
     // one 32-row wave per SIMD (the accumulators need the whole register
@@ -1702,6 +1729,7 @@ hipError_t launch_attention(const LaunchPlan& p, AttnArgs& a, hipStream_t st) {
     if (p.kernel != KERNEL_STREAMS) a.ticket = nullptr;  // (the others always merge in a second kernel)
     hipError_t e = p.kernel == KERNEL_STREAMS ? launch_ring(p, a, st)
                    : p.kernel == KERNEL_HILO  ? launch_hilo(p, a, st)
+                   : p.rows                   ? launch_rows(p, a, st)
                                               : launch_shape(p, a, st);
     if (e != hipSuccess || p.n_split <= 1 || a.ticket) return e;
     const size_t items = (size_t)a.n_batch * a.n_head_kv * a.part_rows * (p.hd_tile / 4);

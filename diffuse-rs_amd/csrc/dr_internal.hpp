@@ -320,12 +320,13 @@ struct LaunchPlan {
     bool w16;        // two 16-row compute waves per (row block, key group)
     int kernel;      // KernelKind
     int merge;       // set at launch: 0 no split, 1 split_merge_kernel, 2 in-kernel
+    bool rows;       // KERNEL_STAGED: attn_rows_kernel (many query rows)
     bool rotate;     // KERNEL_STREAMS: rotate the row groups' tile walks (RingWaveTiles)
 };
 
 // Attention kernel families.  STAGED: attn_fwd_kernel, the workgroup's waves
 // share super-tiles of K/V staged in LDS (every head dim, mask mode and the
-// Q epilogue).  STREAMS: attn_ring_kernel, head dims 128 and 256, each wave
+// Q epilogue), and attn_rows_kernel, its form for many query rows.  STREAMS: attn_ring_kernel, head dims 128 and 256, each wave
 // streams its own key tiles (no mask or MASK_POS, Q norm only).  HILO:
 // attn_hilo_kernel, f32-accurate scores and values from bf16 hi/lo halves of
 // Q, K and V (layers whose cache holds the lo halves, and the drop-in; every
@@ -377,6 +378,7 @@ bool ring_waves_built(int hd, int waves);
 int ring_merge_splits(int hd);  // most key splits attn_ring_kernel merges in-kernel
 hipError_t launch_hilo(const LaunchPlan& p, const AttnArgs& a, hipStream_t st);
 int hilo_rows();  // query rows per workgroup of attn_hilo_kernel
+hipError_t launch_rows(const LaunchPlan& p, const AttnArgs& a, hipStream_t st);
 hipError_t launch_hilo32(const LaunchPlan& p, const AttnArgs& a, hipStream_t st);
 int hilo32_rows(int hd_tile);  // the same of attn_hilo32_kernel (0: head dim not built)
 hipError_t launch_store(int hd_tile, const StoreArgs& a, hipStream_t st);
