@@ -31,6 +31,8 @@
 //   2 KV heads, hd 512, 256 rows x 4352 keys                168.2 -> 133.6 us
 //   8 KV heads, hd 256, window 1024, causal prompt of 4096
 //   and 256 canvas rows (every row asks)                    535.6 -> 324.9 us
+// and, with the run store, by reading Q and writing the rows through LDS
+//   47.3 -> 44.2, 125.4 -> 122.7 and 254.9 -> 243.0 us.
 // A tile of 128 rows and 32 keys takes 2.35 us per CU at head dim 256 (1140
 // TFLOP/s over the chip, where a 8192^3 bf16 matrix product reaches 1280),
 // 2.4-3.2 us per 64 rows at 512; splitting the accumulator in two, reading
@@ -67,6 +69,7 @@ struct Hilo32Geom {
     static constexpr int XCH_F = DSPLIT > 1 ? NW * 16 * 64 : 0;  // floats of the score exchange
     static constexpr size_t LDS_BYTES = (size_t)NBUF * 4 * TILE_B + (size_t)XCH_F * 4;
     static_assert(DMAW == NST / 2 * DSPLIT, "one DMA of K and of V^T per step (two at hd 512)");
+    static_assert(NW * 32 * 1024 <= LDS_BYTES, "the output turns in the tiles' LDS");
     static_assert(LDS_BYTES <= 159 * 1024, "LDS budget");
 };
 
@@ -84,6 +87,20 @@ __device__ __forceinline__ void dma16_asm(__amdgpu_buffer_rsrc_t r, uint32_t lds
         "buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds),
         "v"(voff), "s"(r), "s"(soff)
         : "memory");
+#endif
+}
+
+// a + (16 lanes away) in the even rows of 16 lanes, b + the same in the odd
+// ones
+__device__ __forceinline__ double swap_add16(double a, double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const uint64_t ua = __builtin_bit_cast(uint64_t, a), ub = __builtin_bit_cast(uint64_t, b);
+    const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)ua, (uint32_t)ub, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(ua >> 32), (uint32_t)(ub >> 32), false, false);
+    return __builtin_bit_cast(double, (uint64_t)lo[0] | ((uint64_t)hi[0] << 32)) +
+           __builtin_bit_cast(double, (uint64_t)lo[1] | ((uint64_t)hi[1] << 32));
+#else
+    return a + b;
 #endif
 }
 
@@ -210,102 +227,156 @@ __global__ __launch_bounds__(Hilo32Geom<HD>::NT) void attn_hilo32_kernel(const A
     auto dma_v = [&](int j, int t, int buf) __attribute__((always_inline)) {
         dma16_asm(rv, lds0 + V_OFF + buf * 2 * TILE_B + dma_lds + j * 1024, vvo, t * TILE_B + j * 1024);
     };
-    // the first tiles are requested before Q is read
+    // the first K tiles are requested before Q is read (Q passes through
+    // V^T's part of LDS, so V^T follows it)
     if (t0 < t1) {
 #pragma unroll
         for (int j = 0; j < DMAW; ++j) dma_k(j, t0, 0);
         if constexpr (NBUF == 2) {
-#pragma unroll
-            for (int j = 0; j < DMAW; ++j) dma_v(j, t0, 0);
             const int t = min(t0 + 1, t1 - 1);
 #pragma unroll
             for (int j = 0; j < DMAW; ++j) dma_k(j, t, 1);
         }
     }
 
-    // ---- Q of this lane's row at head dims dim(st) + 8 hf + (0..7): bias,
-    // QK-norm and RoPE (forward.rs:291-310), then hi and lo bf16 halves of
-    // q * scale * log2 e.  A wave's dims are two runs half the head dim
-    // apart, so a dim and its rotary partner sit in one lane (steps st and
-    // st + 8).
+    // ---- Q: bias, QK-norm and RoPE (forward.rs:291-310), then the hi and lo
+    // bf16 halves of q * scale * log2 e as MFMA operands: lane (col, hf) holds
+    // row col at head dims dim(st) + 8 hf + (0..7).  Loaded in that layout
+    // each instruction touches 32 rows, and Q took 8 of the 34 us of C5's
+    // sliding layer.  So 32 lanes read a row (two rows per instruction, lane
+    // l32 the dims 4 l32 .. + 3 of each 128, a dim's rotary partner d + HD / 2
+    // among them), finish it there and pass the halves through LDS, 16 rows
+    // of a row block at a time.  The waves of a split row block finish half
+    // of its rows each.  (16-byte chunk c of a row's half sits at chunk c ^
+    // (row & 15): the operand reads are conflict-free.)
     auto dim = [&](int st) __attribute__((always_inline)) { return (st / 8) * (HD / 2) + dh * 128 + 16 * (st % 8); };
     bf16x8 qh[NST], ql[NST];
     {
-        const size_t head = (size_t)(g * a.group + hg) * HD;
-        const float* qrow = static_cast<const float*>(S.q) + (size_t)qi * a.q_rstride + head;
-        f32x4 x[NST][2];
+        constexpr int NP = 8 / DSPLIT, NPC = HD / 128;  // row pairs per wave and pass, 128-dim pieces
+        const int l32 = lane & 31;
+        char* const qlds = lds + V_OFF + rbw * 16 * (HD * 4);  // [16 rows][hi, lo][HD] bf16
+        f32x4 w[NPC];  // the QK-norm's gains, loaded with the rows
 #pragma unroll
-        for (int st = 0; st < NST; ++st) {
-            const int d0 = dim(st) + 8 * hf;
-            x[st][0] = gload<f32x4>(qrow + d0);
-            x[st][1] = gload<f32x4>(qrow + d0 + 4);
-        }
-        if (a.qb) {
+        for (int c = 0; c < NPC; ++c) w[c] = a.qn_w ? gload<f32x4>(a.qn_w + 128 * c + 4 * l32) : f32x4{};
 #pragma unroll
-            for (int st = 0; st < NST; ++st) {
-                const int d0 = dim(st) + 8 * hf;
-                x[st][0] += gload<f32x4>(a.qb + head + d0);
-                x[st][1] += gload<f32x4>(a.qb + head + d0 + 4);
+        for (int st = 0; st < NST; ++st) qh[st] = ql[st] = bf16x8{};
+#pragma unroll 1  // (half the code: the prologue is straight-line and runs once)
+        for (int pass = 0; pass < 2; ++pass) {
+            const int i0 = 16 * pass + dh * 2 * NP;  // first row of this wave
+            f32x4 x[NP][NPC], tab[NP][NPC];          // (pieces c and c + NPC / 2 share tab[.][2 c], [2 c + 1])
+            int head[NP];
+#pragma unroll
+            for (int k = 0; k < NP; ++k) {  // this lane's row of pair k: i0 + 2 k + hf
+                const int ri = __shfl(qi, i0 + 2 * k + hf);
+                head[k] = (g * a.group + __shfl(hg, i0 + 2 * k + hf)) * HD;
+                const float* row = static_cast<const float*>(S.q) + (size_t)ri * a.q_rstride + head[k] + 4 * l32;
+#pragma unroll
+                for (int c = 0; c < NPC; ++c) x[k][c] = gload<f32x4>(row + 128 * c);
             }
-        }
-        // rms_norm_inplace (ops.rs:106-114): f32 squares summed in f64 over
-        // the row's lanes, half 0's sum first on both waves of a split row
-        if (a.qn_w) {
-            double ss = 0.0;
+            if (a.rope) {  // full rotary: rot == HD (the host checks); pairs 128 c + 4 l32 .. + 3
 #pragma unroll
-            for (int st = 0; st < NST; ++st)
+                for (int k = 0; k < NP; ++k) {
+                    const float* t = a.rope + (size_t)__shfl(my_qpos, i0 + 2 * k + hf) * HD + 8 * l32;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float v = x[st][e >> 2][e & 3];
-                    const float sq = v * v;
-                    ss += (double)sq;
-                }
-            ss += __shfl_xor(ss, 32);
-            if constexpr (DSPLIT > 1) {
-                __shared__ double s_ss[NW][32];
-                if (hf == 0) s_ss[wave][col] = ss;
-                lds_barrier();
-                const double other = s_ss[wave ^ RBW][col];
-                ss = dh == 0 ? ss + other : other + ss;
-            }
-            const float sc = 1.0f / (float)sqrt(ss / (double)HD + (double)a.qn_eps);
-#pragma unroll
-            for (int st = 0; st < NST; ++st) {
-                const int d0 = dim(st) + 8 * hf;
-                const f32x4 w0 = gload<f32x4>(a.qn_w + d0), w1 = gload<f32x4>(a.qn_w + d0 + 4);
-                {
-#pragma clang fp contract(off)
-                    x[st][0] = x[st][0] * sc * w0;
-                    x[st][1] = x[st][1] * sc * w1;
+                    for (int c = 0; c < NPC; ++c) tab[k][c] = gload<f32x4>(t + 256 * (c / 2) + 4 * (c & 1));
                 }
             }
-        }
-        if (a.rope) {  // full rotary: rot == HD (the host checks)
-            const float* tab = a.rope + (size_t)my_qpos * HD;  // [HD / 2] (sin, cos)
+            if (a.qb) {
 #pragma unroll
-            for (int st = 0; st < NST / 2; ++st)
+                for (int k = 0; k < NP; ++k)
 #pragma unroll
-                for (int p = 0; p < 2; ++p) {
-                    const int d0 = dim(st) + 8 * hf + 4 * p;
-                    const f32x4 t0v = gload<f32x4>(tab + 2 * d0), t1v = gload<f32x4>(tab + 2 * d0 + 4);
-                    const float sn[4] = {t0v[0], t0v[2], t1v[0], t1v[2]}, cs[4] = {t0v[1], t0v[3], t1v[1], t1v[3]};
+                    for (int c = 0; c < NPC; ++c) x[k][c] += gload<f32x4>(a.qb + head[k] + 128 * c + 4 * l32);
+            }
+            // rms_norm_inplace (ops.rs:106-114): f32 squares summed in f64.
+            // The rows' sums meet across their 32 lanes together: at each step
+            // a lane gives away half of its rows' sums and keeps the rest, so
+            // lane (hf, l32) ends up with the sum of pair l32 / (32 / NP).
+            if (a.qn_w) {
+                double ss[NP];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float lo = x[st][p][e], hi = x[st + NST / 2][p][e];
-                        x[st][p][e] = rope_lo(lo, hi, sn[e], cs[e]);
-                        x[st + NST / 2][p][e] = rope_hi(lo, hi, sn[e], cs[e]);
+                for (int k = 0; k < NP; ++k) {
+                    ss[k] = 0.0;
+#pragma unroll
+                    for (int e = 0; e < 4 * NPC; ++e) {
+                        const float v = x[k][e >> 2][e & 3];
+                        const float sq = v * v;
+                        ss[k] += (double)sq;
                     }
                 }
-        }
 #pragma unroll
-        for (int st = 0; st < NST; ++st)
+                for (int k = 0; k < NP / 2; ++k) ss[k] = swap_add16(ss[k], ss[k + NP / 2]);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float xs = rvalid ? x[st][e >> 2][e & 3] * a.c : 0.0f;
-                const __bf16 h = (__bf16)xs;
-                qh[st][e] = h;
-                ql[st][e] = (__bf16)(xs - (float)h);
+                for (int k = 0; k < NP / 4; ++k) {
+                    const bool up = (lane & 8) != 0;
+                    const double give = up ? ss[k] : ss[k + NP / 4], keep = up ? ss[k + NP / 4] : ss[k];
+                    ss[k] = keep + __shfl_xor(give, 8);
+                }
+                if constexpr (NP == 8) {
+                    const bool up = (lane & 4) != 0;
+                    const double give = up ? ss[0] : ss[1], keep = up ? ss[1] : ss[0];
+                    ss[0] = keep + __shfl_xor(give, 4);
+                } else {
+                    ss[0] += __shfl_xor(ss[0], 4);
+                }
+                ss[0] += __shfl_xor(ss[0], 2);
+                ss[0] += __shfl_xor(ss[0], 1);
+                const float sc = 1.0f / (float)sqrt(ss[0] / (double)HD + (double)a.qn_eps);
+#pragma unroll
+                for (int k = 0; k < NP; ++k) {
+#pragma clang fp contract(off)
+                    const float rs = __shfl(sc, (lane & 32) + k * (32 / NP));
+#pragma unroll
+                    for (int c = 0; c < NPC; ++c) x[k][c] = x[k][c] * rs * w[c];
+                }
             }
+            if (a.rope) {
+#pragma unroll
+                for (int k = 0; k < NP; ++k)
+#pragma unroll
+                    for (int c = 0; c < NPC / 2; ++c)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float sn = tab[k][2 * c + (e >> 1)][2 * (e & 1)];
+                            const float cs = tab[k][2 * c + (e >> 1)][2 * (e & 1) + 1];
+                            const float lo = x[k][c][e], hi = x[k][c + NPC / 2][e];
+                            x[k][c][e] = rope_lo(lo, hi, sn, cs);
+                            x[k][c + NPC / 2][e] = rope_hi(lo, hi, sn, cs);
+                        }
+            }
+            if (pass > 0 && DSPLIT > 1) lds_barrier();  // the first pass's operands are read
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();  // (a wave's own accesses run in order)
+#pragma unroll
+            for (int k = 0; k < NP; ++k) {
+                const int row = dh * 2 * NP + 2 * k + hf;
+                // (rows past the last: finite garbage, never stored)
+                char* const dst = qlds + row * (HD * 4) + (((l32 >> 1) ^ (row & 15)) << 4) + 8 * (l32 & 1);
+#pragma unroll
+                for (int c = 0; c < NPC; ++c) {
+                    bf16x4 h, lo;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float xs = x[k][c][e] * a.c;
+                        h[e] = (__bf16)xs;
+                        lo[e] = (__bf16)(xs - (float)h[e]);
+                    }
+                    *reinterpret_cast<bf16x4*>(dst + 256 * c) = h;
+                    *reinterpret_cast<bf16x4*>(dst + 256 * c + HD * 2) = lo;
+                }
+            }
+            if constexpr (DSPLIT > 1) lds_barrier();
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+            if ((col >> 4) == pass) {
+                const char* src = qlds + (col & 15) * (HD * 4);
+#pragma unroll
+                for (int st = 0; st < NST; ++st) {
+                    const int off = ((dim(st) / 8 + hf) ^ (col & 15)) << 4;
+                    qh[st] = *reinterpret_cast<const bf16x8*>(src + off);
+                    ql[st] = *reinterpret_cast<const bf16x8*>(src + HD * 2 + off);
+                }
+            }
+        }
     }
 
     f32x16 o[NDB];
@@ -464,9 +535,13 @@ __global__ __launch_bounds__(Hilo32Geom<HD>::NT) void attn_hilo32_kernel(const A
     };
 
     if (t0 < t1) {
-        // ---- scores of the first tile (K(t0) is the oldest DMA)
+        // ---- scores of the first tile
         wait_vmcnt<0>();
-        lds_barrier();
+        lds_barrier();  // (and every wave has its Q: V^T may take that part of LDS)
+        if constexpr (NBUF == 2) {
+#pragma unroll
+            for (int j = 0; j < DMAW; ++j) dma_v(j, t0, 0);
+        }
 #pragma unroll
         for (int i = 0; i < 16; ++i) sn[i] = 0.0f;
         {
@@ -491,31 +566,50 @@ __global__ __launch_bounds__(Hilo32Geom<HD>::NT) void attn_hilo32_kernel(const A
         wait_vmcnt<0>();  // (no DMA may outlive the workgroup's LDS)
     }
 
-    // ---- the row's sum over its lane halves; out or the split partial
+    // ---- the row's sum over its lane halves; out or the split partial.
+    // o[db][i] is O^T[d = 256 dh + 32 db + 8 (i / 4) + 4 hf + i % 4][col]: 16
+    // bytes of 32 rows per register quad, so the wave turns its 32 rows x 256
+    // dims in LDS (chunk c of row q at chunk c ^ q) and stores whole rows
+    // (in the register layout the stores of C5's sliding layer, 33 MB of
+    // partials, took 6 of its 34 us).
     l += __shfl_xor(l, 32);
-    if (!rvalid) return;
-    // o[db][i] is O^T[d = 256 dh + 32 db + 8 (i / 4) + 4 hf + i % 4][col]
-    if (a.n_split <= 1) {
-        float* orow = S.out + (size_t)qi * a.o_rstride + (size_t)(g * a.group + hg) * HD + dh * 256 + 4 * hf;
-        const float il = __builtin_amdgcn_rcpf(l);  // no visible key: 0 * inf = NaN (attention.rs:181-185)
+    lds_barrier();  // every wave is done with the tiles
+    char* const rows = lds + wave * 32 * 1024;
+    const float f = a.n_split <= 1 ? __builtin_amdgcn_rcpf(l) : 1.0f;  // no visible key: 0 * inf = NaN (attention.rs:181-185)
 #pragma unroll
-        for (int db = 0; db < NDB; ++db)
+    for (int db = 0; db < NDB; ++db)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                gstore(orow + 32 * db + 8 * j,
-                       f32x4{o[db][4 * j] * il, o[db][4 * j + 1] * il, o[db][4 * j + 2] * il, o[db][4 * j + 3] * il});
-    } else {
-        const size_t plane = (size_t)a.n_batch * a.n_head_kv * a.part_rows;
-        const size_t prow = (size_t)(b * a.n_head_kv + g) * a.part_rows + r;
-        float* po = a.part_o + (size_t)split * plane * HD + prow * HD + dh * 256 + 4 * hf;
+        for (int j = 0; j < 4; ++j) {
+            f32x4 v;
 #pragma unroll
-        for (int db = 0; db < NDB; ++db)
+            for (int e = 0; e < 4; ++e) v[e] = o[db][4 * j + e] * f;
+            *reinterpret_cast<f32x4*>(rows + col * 1024 + (((8 * db + 2 * j + hf) ^ col) << 4)) = v;
+        }
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+    const size_t plane = (size_t)a.n_batch * a.n_head_kv * a.part_rows;
+    const size_t prow0 = (size_t)(b * a.n_head_kv + g) * a.part_rows + wg_row0 + rbw * 32;
+    const int nrow = min(32, rows_total - wg_row0 - rbw * 32);
+#pragma unroll 1
+    for (int i0 = 0; i0 < nrow; i0 += 8) {
+        f32x4 v[8];
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                gstore(po + 32 * db + 8 * j,
-                       f32x4{o[db][4 * j], o[db][4 * j + 1], o[db][4 * j + 2], o[db][4 * j + 3]});
-        if (dh == 0 && hf == 0) gstore(a.part_ml + ((size_t)split * plane + prow) * 2, make_float2(m, l));
+        for (int k = 0; k < 8; ++k)
+            v[k] = *reinterpret_cast<const f32x4*>(rows + (i0 + k) * 1024 + ((lane ^ (i0 + k)) << 4));
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            float* dst;
+            if (a.n_split <= 1) {
+                const int ri = __builtin_amdgcn_readlane(qi, i0 + k), rh = __builtin_amdgcn_readlane(hg, i0 + k);
+                dst = S.out + (size_t)ri * a.o_rstride + (size_t)(g * a.group + rh) * HD;
+            } else {
+                dst = a.part_o + ((size_t)split * plane + prow0 + i0 + k) * HD;
+            }
+            if (i0 + k < nrow) gstore(dst + dh * 256 + 4 * lane, v[k]);
+        }
     }
+    if (a.n_split > 1 && rvalid && dh == 0 && hf == 0)
+        gstore(a.part_ml + ((size_t)split * plane + prow0 + col) * 2, make_float2(m, l));
 }
 
 template <int HD>
