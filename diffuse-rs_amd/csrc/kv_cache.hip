@@ -16,9 +16,9 @@
 //         ops.rs:384-389, applied before the store in forward.rs:300-302).
 //         A layer kept at hi/lo precision also gets the lo halves,
 //         bf16(x - bf16(x)), of K and V in planes laid out like K and V^T.
-//         One launch.  Rows at contiguous positions (canvas, prompt): one
-//         workgroup per (kv head, 32-key tile), whole-line loads and stores.
-//         Position lists and padded head dims: one workgroup per (64-row
+//         One launch.  Rows at contiguous positions (canvas, prompt) or at
+//         a position list: one workgroup per (kv head, 32 rows, K or V),
+//         whole-line loads.  Padded head dims: one workgroup per (64-row
 //         block, 64-wide head-dim chunk, kv head), K converted in registers,
 //         V transposed through LDS.
 // gather: StepCache::gather (cache.rs:73-82) -- bf16 back to f32 rows (hi +
@@ -439,8 +439,8 @@ __global__ __launch_bounds__(256) void kv_store_tiles_kernel(const StoreArgs a) 
     }
 }
 
-// The store of rows at contiguous positions, head dim == HD: the canvas rows
-// of a denoise step, the prompt, a first pass.  One workgroup per (kv head,
+// The store of rows at contiguous positions or at a sorted position list, head
+// dim == HD: the rows of a denoise step, the prompt, a first pass.  One workgroup per (kv head,
 // 32-key tile that the rows touch, K or V); rows need not fill the first and
 // the last tile.  K and V take a workgroup each, so a step's few tiles give
 // twice the workgroups, each with half the loads to wait for.
@@ -462,8 +462,11 @@ __global__ __launch_bounds__(256) void kv_store_tiles_kernel(const StoreArgs a) 
 // 512 before: see the figures at launch_store.
 // EPI: biases, norms and RoPE are compiled in (the plain build keeps them
 // out: its stores then wait for their own loads only).  HILO: the lo planes
-// are written too.
-template <int HD, bool EPI, bool HILO>
+// are written too.  LIST: the rows go to the positions of a sorted list
+// (split_active's rows), 32 rows of the list per workgroup; V is turned in
+// LDS, so that a store instruction's 2-byte writes are 32 rows of two d-rows
+// and fall into the few 32-key tiles that sorted positions span.
+template <int HD, bool EPI, bool HILO, bool LIST>
 __global__ __launch_bounds__(HD) void kv_store_run_kernel(const StoreArgs a) {
     constexpr int RPG = 4, NRG = VT_KEYS / RPG;  // rows per thread, row groups
     constexpr int NWV = HD / 64;                 // waves
@@ -473,10 +476,16 @@ __global__ __launch_bounds__(HD) void kv_store_run_kernel(const StoreArgs a) {
     if (lid >= a.n_head_kv * a.n_rb * 2) return;
     const int g = lid / (2 * a.n_rb), rest = lid - g * 2 * a.n_rb;
     const bool is_v = rest & 1;
-    const int kt = a.pos0 / VT_KEYS + (rest >> 1);  // key tile
+    const int kt = LIST ? 0 : a.pos0 / VT_KEYS + (rest >> 1);  // key tile
     const int tid = threadIdx.x, rg = tid % NRG, dc = tid / NRG;
     const int p0 = kt * VT_KEYS + rg * RPG;  // first position of this thread
-    const int r0 = p0 - a.pos0;              // its row (rows outside [0, n) are not stored)
+    // its first row (rows outside [0, n) are not stored)
+    const int r0 = LIST ? (rest >> 1) * VT_KEYS + rg * RPG : p0 - a.pos0;
+    int lp[RPG];  // LIST: the rows' positions
+    if constexpr (LIST) {
+#pragma unroll
+        for (int j = 0; j < RPG; ++j) lp[j] = a.pos[min(r0 + j, a.n - 1)];
+    }
     const float* src = (is_v ? a.v : a.k) + (size_t)g * HD + 4 * dc;
     f32x4 xa[RPG], xb[RPG];  // dims 4 dc .., dims HD / 2 + 4 dc ..
 #pragma unroll
@@ -496,7 +505,7 @@ __global__ __launch_bounds__(HD) void kv_store_run_kernel(const StoreArgs a) {
             const int jj = d0 < half ? d0 : d0 - half;
 #pragma unroll
             for (int j = 0; j < RPG; ++j) {
-                const int pos = a.pos0 + min(max(r0 + j, 0), a.n - 1);
+                const int pos = LIST ? lp[j] : a.pos0 + min(max(r0 + j, 0), a.n - 1);
                 const float* e = a.rope + ((size_t)pos * half + jj) * 2;
                 t[j][0] = *reinterpret_cast<const f32x4*>(e);
                 t[j][1] = *reinterpret_cast<const f32x4*>(e + 4);
@@ -591,16 +600,38 @@ __global__ __launch_bounds__(HD) void kv_store_run_kernel(const StoreArgs a) {
     // the bf16 halves: hi, and lo = bf16 of what that rounding dropped
     auto put = [&](uint16_t* plane, auto conv) __attribute__((always_inline)) {
         if (!is_v) {
-            uint16_t* dst = plane + ((size_t)g * a.cap + p0) * HD + 4 * dc;
+            uint16_t* head = plane + (size_t)g * a.cap * HD + 4 * dc;
 #pragma unroll
             for (int j = 0; j < RPG; ++j) {
                 if (r0 + j < 0 || r0 + j >= a.n) continue;
-                *reinterpret_cast<uint2*>(dst + (size_t)j * HD) =
+                uint16_t* dst = head + (size_t)(LIST ? lp[j] : p0 + j) * HD;
+                *reinterpret_cast<uint2*>(dst) =
                     make_uint2((uint32_t)conv(xa[j][0]) | ((uint32_t)conv(xa[j][1]) << 16),
                                (uint32_t)conv(xa[j][2]) | ((uint32_t)conv(xa[j][3]) << 16));
-                *reinterpret_cast<uint2*>(dst + (size_t)j * HD + HD / 2) =
+                *reinterpret_cast<uint2*>(dst + HD / 2) =
                     make_uint2((uint32_t)conv(xb[j][0]) | ((uint32_t)conv(xb[j][1]) << 16),
                                (uint32_t)conv(xb[j][2]) | ((uint32_t)conv(xb[j][3]) << 16));
+            }
+            return;
+        }
+        if constexpr (LIST) {
+            __shared__ __align__(8) uint16_t s_v[HD][VT_KEYS + 4];
+            __syncthreads();  // (the lo plane's turn: the hi values are read)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                uint16_t h[RPG];
+#pragma unroll
+                for (int j = 0; j < RPG; ++j) h[j] = conv(e < 4 ? xa[j][e & 3] : xb[j][e & 3]);
+                *reinterpret_cast<uint2*>(&s_v[(e < 4 ? 0 : HD / 2) + 4 * dc + (e & 3)][rg * RPG]) =
+                    make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+            }
+            __syncthreads();
+            const int row = tid % VT_KEYS, r = (rest >> 1) * VT_KEYS + row;
+            if (r < a.n) {
+                const int pos = a.pos[r];
+                uint16_t* dst = plane + (size_t)g * HD * a.cap + (size_t)(pos / VT_KEYS) * (HD * VT_KEYS) + pos % VT_KEYS;
+#pragma unroll 8
+                for (int d = tid / VT_KEYS; d < HD; d += HD / VT_KEYS) dst[(size_t)d * VT_KEYS] = s_v[d][row];
             }
             return;
         }
@@ -645,18 +676,18 @@ __global__ __launch_bounds__(256) void kv_gather_kernel(const GatherArgs a) {
     }
 }
 
-template <int HD>
+template <int HD, bool LIST>
 void launch_run(const StoreArgs& a, bool epi, dim3 grid, hipStream_t st) {
     if (a.klo) {
         if (epi)
-            hipLaunchKernelGGL((kv_store_run_kernel<HD, true, true>), grid, dim3(HD), 0, st, a);
+            hipLaunchKernelGGL((kv_store_run_kernel<HD, true, true, LIST>), grid, dim3(HD), 0, st, a);
         else
-            hipLaunchKernelGGL((kv_store_run_kernel<HD, false, true>), grid, dim3(HD), 0, st, a);
+            hipLaunchKernelGGL((kv_store_run_kernel<HD, false, true, LIST>), grid, dim3(HD), 0, st, a);
     } else {
         if (epi)
-            hipLaunchKernelGGL((kv_store_run_kernel<HD, true, false>), grid, dim3(HD), 0, st, a);
+            hipLaunchKernelGGL((kv_store_run_kernel<HD, true, false, LIST>), grid, dim3(HD), 0, st, a);
         else
-            hipLaunchKernelGGL((kv_store_run_kernel<HD, false, false>), grid, dim3(HD), 0, st, a);
+            hipLaunchKernelGGL((kv_store_run_kernel<HD, false, false, LIST>), grid, dim3(HD), 0, st, a);
     }
 }
 
@@ -675,8 +706,9 @@ hipError_t launch_store(int hd_tile, const StoreArgs& args, hipStream_t st) {
     a.xcd_n = std::max(1, 8 * (a.batch + 1) / nb - a.xcd_lo);
     // Rows at contiguous positions whose head dim fills its tile: the tile
     // kernel where they are whole tiles to be stored as they are, else the
-    // run kernel.  Position lists, padded head dims, rows that are not 16-byte
-    // aligned and a partial rotary at head dim 512 take the general kernel.
+    // run kernel, which also takes position lists.  Padded head dims, rows that
+    // are not 16-byte aligned and a partial rotary at head dim 512 take the
+    // general kernel.
     // Run kernel against the kernels that took these calls before (general;
     // * the tile kernel with an epilogue), in us, kernel times:
     //   16 heads, hd 128, 512 rows from position 2041, norm + RoPE   12.5 / 7.0
@@ -685,12 +717,14 @@ hipError_t launch_store(int hd_tile, const StoreArgs& args, hipStream_t st) {
     //   8 heads, hd 256, 4352 rows, hi/lo, norms + RoPE               121 / 47.7
     //   4 heads, hd 128, 1280 rows, bias + RoPE *                     7.8 / 6.5
     //   32 heads, hd 128, 64 rows, RoPE *                             5.1 / 4.0
+    //   32 heads, hd 128, 145 listed rows of 256 positions, RoPE      8.2 / 5.6
+    //   the same, 404 of 512                                         12.1 / 9.0
     const int p0 = a.pos0 >= 0 ? a.pos0 : (a.pos == nullptr ? 0 : -1);
     const bool rot_ok = !a.rope || a.rot == a.hd || (hd_tile <= 256 && a.rot % 8 == 0 && a.rot <= a.hd);
-    const bool run = a.vec && a.hd == hd_tile && p0 >= 0 && rot_ok && !a.klo == !a.vlo &&
+    const bool run = a.vec && a.hd == hd_tile && rot_ok && !a.klo == !a.vlo &&
                      (((uintptr_t)a.kn_w | (uintptr_t)a.kb | (uintptr_t)a.vb | (uintptr_t)a.rope) & 15) == 0;
     const bool epi = a.kn_w || a.kb || a.vb || a.v_norm || a.rope;
-    if (run && !epi && !a.klo && hd_tile <= 256 && p0 % VT_KEYS == 0 && a.n % VT_KEYS == 0) {
+    if (run && p0 >= 0 && !epi && !a.klo && hd_tile <= 256 && p0 % VT_KEYS == 0 && a.n % VT_KEYS == 0) {
         a.pos0 = p0;
         const int work = a.n_head_kv * (a.n / VT_KEYS);
         a.per_xcd = (work + a.xcd_n - 1) / a.xcd_n;
@@ -703,16 +737,21 @@ hipError_t launch_store(int hd_tile, const StoreArgs& args, hipStream_t st) {
         return hipGetLastError();
     }
     if (run) {
+        const bool list = p0 < 0;
         a.pos0 = p0;
-        a.n_rb = (p0 + a.n - 1) / VT_KEYS - p0 / VT_KEYS + 1;
+        a.n_rb = list ? (a.n + VT_KEYS - 1) / VT_KEYS : (p0 + a.n - 1) / VT_KEYS - p0 / VT_KEYS + 1;
         const int work = a.n_head_kv * a.n_rb * 2;
         a.per_xcd = (work + a.xcd_n - 1) / a.xcd_n;
         const dim3 grid((unsigned)(8 * a.per_xcd));
-        switch (hd_tile) {
-            case 64: launch_run<64>(a, epi, grid, st); break;
-            case 128: launch_run<128>(a, epi, grid, st); break;
-            case 256: launch_run<256>(a, epi, grid, st); break;
-            default: launch_run<512>(a, epi, grid, st); break;
+        switch (hd_tile * 2 + (list ? 1 : 0)) {
+            case 128: launch_run<64, false>(a, epi, grid, st); break;
+            case 129: launch_run<64, true>(a, epi, grid, st); break;
+            case 256: launch_run<128, false>(a, epi, grid, st); break;
+            case 257: launch_run<128, true>(a, epi, grid, st); break;
+            case 512: launch_run<256, false>(a, epi, grid, st); break;
+            case 513: launch_run<256, true>(a, epi, grid, st); break;
+            case 1024: launch_run<512, false>(a, epi, grid, st); break;
+            default: launch_run<512, true>(a, epi, grid, st); break;
         }
         return hipGetLastError();
     }
