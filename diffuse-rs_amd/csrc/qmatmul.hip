@@ -800,7 +800,7 @@ __global__ __launch_bounds__(512) void qmm0_kernel(const QmmArgs a) {
 // of 32 activation rows: a wave forms its own weight operands (no wave
 // shares them, so the loop has no barrier), keeps several blocks' loads in
 // flight and uses each operand for TT tiles.  The eighths meet in LDS and are
-// added in their order, so every output is summed in one fixed order.
+// added in pairs, so every output is summed in one fixed order.
 // 1024 x 2048 Q8_0 weights, up to 32 rows, kernel alone: 14.2 -> 6.1 us; 64
 // rows 8.4.
 template <int TT>
@@ -818,12 +818,16 @@ __device__ __forceinline__ void finish_slices(const QmmArgs& a, const f32x16 (&s
         for (int k = 0; k < 2; ++k) {
             const int i = wave + 8 * k;
             const int t = t0 + 32 * tt + 8 * (i >> 2) + 4 * g + (i & 3);
-            float v = s_red[0][i][lane];
+            // (pairwise, 6.5e-8 from 64 bits at Q6_K 2048 x 4096: adding the
+            // eighths one after the other rounds more, 6.8e-8, than the two
+            // halves of the walking kernels, 6.6e-8)
+            float v[8];
 #pragma unroll
-            for (int w = 1; w < 8; ++w) v = v + s_red[w][i][lane];
+            for (int w = 0; w < 8; ++w) v[w] = s_red[w][i][lane];
+            float y = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
             if (t < a.n && rr < a.rows) {
-                if (a.residual) v += gld<float>(a.residual + (size_t)t * a.rows + rr);
-                a.out[(size_t)t * a.rows + rr] = v;
+                if (a.residual) y += gld<float>(a.residual + (size_t)t * a.rows + rr);
+                a.out[(size_t)t * a.rows + rr] = y;
             }
         }
     }
