@@ -808,6 +808,18 @@ __device__ __forceinline__ void finish_slices(const QmmArgs& a, const f32x16 (&s
                                               int wave, int lane, int t0, int rt) {
     const int c = lane & 31, g = lane >> 5;
     const int rr = rt * 32 + c;
+    auto row = [&](int tt, int k) __attribute__((always_inline)) {
+        const int i = wave + 8 * k;
+        return t0 + 32 * tt + 8 * (i >> 2) + 4 * g + (i & 3);
+    };
+    float rv[TT][2];  // (every index in bounds, so that all are in flight together: see load_residual)
+    if (a.residual) {
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+                rv[tt][k] = gld<float>(a.residual + (size_t)min(row(tt, k), a.n - 1) * a.rows + min(rr, a.rows - 1));
+    }
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
         if (tt > 0) lds_barrier();  // the tile before is read
@@ -816,17 +828,16 @@ __device__ __forceinline__ void finish_slices(const QmmArgs& a, const f32x16 (&s
         lds_barrier();
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
-            const int i = wave + 8 * k;
-            const int t = t0 + 32 * tt + 8 * (i >> 2) + 4 * g + (i & 3);
             // (pairwise, 6.5e-8 from 64 bits at Q6_K 2048 x 4096: adding the
             // eighths one after the other rounds more, 6.8e-8, than the two
             // halves of the walking kernels, 6.6e-8)
             float v[8];
 #pragma unroll
-            for (int w = 0; w < 8; ++w) v[w] = s_red[w][i][lane];
+            for (int w = 0; w < 8; ++w) v[w] = s_red[w][wave + 8 * k][lane];
             float y = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+            const int t = row(tt, k);
             if (t < a.n && rr < a.rows) {
-                if (a.residual) y += gld<float>(a.residual + (size_t)t * a.rows + rr);
+                if (a.residual) y += rv[tt][k];
                 a.out[(size_t)t * a.rows + rr] = y;
             }
         }
