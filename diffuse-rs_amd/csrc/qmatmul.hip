@@ -237,7 +237,7 @@ __global__ __launch_bounds__(512) void q8k_quantize_tiles_kernel(const float* __
 // slab s of row c; accumulator slot i of that lane is output (t = 8 (i / 4) +
 // 4 g + i % 4, r = c).
 //
-// (This kernel runs Q4_K only; Q6_K always takes qmm_slice_kernel below.)
+// (This kernel runs Q4_K only; Q6_K always takes qmm6_slice_kernel below.)
 // Weight operand of a Q4_K block: slab s = sub-block s.  sc_s = 8 sh + sl with
 // sh, sl <= 7, so sh * q and sl * q (q <= 15) are bytes and a 16-bit packed
 // multiply scales two nibble bytes at once without carries; the two parts
@@ -271,17 +271,6 @@ __device__ __forceinline__ void load_raw(const uint8_t* blk, int c, int g, RawBl
     r.h = gld<u32x4>(blk);
     r.q = gld<u32x4>(blk + 16 + 32 * c + 16 * g);
 }
-// slabs 2 c, 2 c + 1 of a Q6_K block: half c / 2, quarters 2 (c % 2), + 1
-// (src/kernels.rs:135-147): ql runs 64 h + 32 a + 16 g, qh run 32 h + 16 g
-__device__ __forceinline__ void load_raw(const uint8_t* blk, int c, int g, RawBlock<14>& r) {
-    const int h = c >> 1;
-    r.sc = gld16_a2(blk + 192);
-    r.ql[0] = gld16_a2(blk + 64 * h + 16 * g);
-    r.ql[1] = gld16_a2(blk + 64 * h + 32 + 16 * g);
-    r.qh = gld16_a2(blk + 128 + 32 * h + 16 * g);
-    r.d = gld<uint16_t>(blk + 208);
-}
-
 // What the combine of a block needs besides the MFMA results.
 struct BlockScale {
     float wd, wdmin;
@@ -972,14 +961,13 @@ __global__ __launch_bounds__(512) void qmm0_slice_kernel(const QmmArgs a) {
     finish_slices<TT>(a, sum, *reinterpret_cast<float(*)[8][16][64]>(s_mem), wave, lane, t32 * 32, rt);
 }
 
-// The k-quants.  A wave forms the weight operands of its block two slabs at a
+// Q4_K.  A wave forms the weight operands of its block two slabs at a
 // time (prep of the kernel above, into registers) and multiplies them with
 // every tile; the hi and lo parts run as two accumulators.
-template <int WT, int TT>
+template <int TT>
 __global__ __launch_bounds__(512) void qmm_slice_kernel(const QmmArgs a) {
-    constexpr bool Q4 = WT == 12;
-    constexpr int WB = Q4 ? Q4K_BYTES : Q6K_BYTES;
-    constexpr int SHIFT = Q4 ? 3 : 6;
+    constexpr int WB = Q4K_BYTES;
+    constexpr int SHIFT = 3;
     __shared__ float s_red[8][16][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -994,7 +982,7 @@ __global__ __launch_bounds__(512) void qmm_slice_kernel(const QmmArgs a) {
     const int b0 = min(wave * per, nb), cnt = min(b0 + per, nb) - b0;
     const int blast = cnt > 0 ? b0 + cnt - 1 : nb - 1;
     struct Stage {
-        RawBlock<WT> raw[4];  // slabs 2 k, 2 k + 1 (what they share is loaded once: the compiler sees equal addresses)
+        RawBlock<12> raw[4];  // slabs 2 k, 2 k + 1 (what they share is loaded once: the compiler sees equal addresses)
         i32x4 av[TT][8];
         float xd[TT];
         bf16x8 bm[TT];
@@ -1009,7 +997,7 @@ __global__ __launch_bounds__(512) void qmm_slice_kernel(const QmmArgs a) {
             for (int s = 0; s < 8; ++s)
                 st.av[tt][s] = gld<i32x4>(L.qs + (((size_t)(t32 + tt) * nb + b) * 8 + s) * 1024 + lane * 16);
             st.xd[tt] = gld<float>(L.xd + ((size_t)(t32 + tt) * nb + b) * 32 + c);
-            if constexpr (Q4) st.bm[tt] = gld<bf16x8>(L.bmin + (((size_t)(t32 + tt) * nb + b) * 64 + lane) * 8);
+            st.bm[tt] = gld<bf16x8>(L.bmin + (((size_t)(t32 + tt) * nb + b) * 64 + lane) * 8);
         }
     };
     f32x16 sum[TT];
@@ -1050,15 +1038,13 @@ __global__ __launch_bounds__(512) void qmm_slice_kernel(const QmmArgs a) {
             const float xa = g == 0 ? cur.xd[tt] : 0.0f;
             const f32x16 dd = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, g == 0 ? bsc.wd : 0.0f, z, 0, 0, 0);
             f32x16 mins = {}, dm = {};
-            if constexpr (Q4) {
-                mins = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.bm[tt], bsc.mn, mins, 0, 0, 0);
-                dm = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, g == 0 ? bsc.wdmin : 0.0f, z, 0, 0, 0);
-            }
+            mins = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.bm[tt], bsc.mn, mins, 0, 0, 0);
+            dm = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, g == 0 ? bsc.wdmin : 0.0f, z, 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const int v = (hi[tt][i] << SHIFT) + lo[tt][i];
                 sum[tt][i] = __builtin_fmaf(dd[i], (float)v, sum[tt][i]);
-                if constexpr (Q4) sum[tt][i] = __builtin_fmaf(-dm[i], mins[i], sum[tt][i]);
+                sum[tt][i] = __builtin_fmaf(-dm[i], mins[i], sum[tt][i]);
             }
         }
     };
@@ -1073,6 +1059,153 @@ __global__ __launch_bounds__(512) void qmm_slice_kernel(const QmmArgs a) {
         for (int it = 0; it < cnt; ++it) block(it, S[0], S[0]);
     }
     finish_slices<TT>(a, sum, s_red, wave, lane, t32 * 32, rt);
+}
+
+// Q6_K.  A block is 210 bytes at any even address: its rows are read as the
+// 32-value types' are, in row order through LDS, one block at a time (read
+// directly, each of 12 loads touched 32 rows, and the address unit was busy
+// for two thirds of the kernel).  Operands of the next block are loaded into
+// the registers whose contents were just used, so every load is a block ahead
+// of its use without a second set of registers.  What bounds it where it is
+// large is forming the operands (VALU) beside the hi and lo products.  4096 x
+// 4096, before / now, us: 20 rows 19.3 / 13.6, 64 16.2 / 15.3, 512 50.9 / 48.1,
+// 2553 225 / 216; 2048 x 4096, 2553 rows with the norm 135 / 130.
+template <int TT>
+__global__ __launch_bounds__(512) void qmm6_slice_kernel(const QmmArgs a) {
+    constexpr int WB = Q6K_BYTES;
+    constexpr int SHIFT = 6;
+    constexpr int NP = (WB + 2 + 15) / 16, NL = (32 * NP + 63) / 64, RS = (NP * 4) | 1;  // (as SliceGeom)
+    constexpr size_t W_BYTES = sizeof(uint32_t) * 8 * 32 * RS, R_BYTES = sizeof(float) * 8 * 16 * 64;
+    __shared__ __align__(16) char s_mem[W_BYTES > R_BYTES ? W_BYTES : R_BYTES];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 31, g = lane >> 5;
+    const int nb = a.cols / QK;
+    const int n_rt = (a.rows + 31) / 32, tg = blockIdx.x / n_rt, rt = blockIdx.x - tg * n_rt;
+    const int t32 = tg * TT;  // first activation tile
+    const QmmLayout L(a.ws, a.n_pad, a.cols);
+    const int per = (nb + 7) / 8;
+    const int b0 = min(wave * per, nb), cnt = min(b0 + per, nb) - b0;
+
+    // pieces of the 32 weight rows, from the 4-byte boundary at or before the first
+    uint32_t* const sw = reinterpret_cast<uint32_t*>(s_mem) + wave * 32 * RS;
+    const uint8_t* w0 = static_cast<const uint8_t*>(a.w) + (size_t)rt * 32 * nb * WB;
+    const int mis0 = (int)((uintptr_t)w0 & 3), row_b = nb * WB;
+    const int bytes = (mis0 + min(32, a.rows - rt * 32) * row_b + 3) & ~3;
+    const __amdgpu_buffer_rsrc_t rw =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w0 - mis0), 0, bytes, 0x00020000);
+    u32x4 pc[NL];
+    auto load_w = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < NL; ++k) {
+            const int idx = k * 64 + lane, row = idx / NP, p = idx - row * NP;
+            const int off = (mis0 + row * row_b + (b0 + j) * WB) & ~3;
+            // (rows past the tile and blocks past the slice: nothing is read)
+            pc[k] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                  rw, row < 32 && j < cnt ? off + 16 * p : bytes, 0, 0));
+        }
+    };
+    auto store_w = [&]() __attribute__((always_inline)) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();  // (the block before is read: LDS runs a wave's accesses in order)
+#pragma unroll
+        for (int k = 0; k < NL; ++k) {
+            const int idx = k * 64 + lane, row = idx / NP, p = idx - row * NP;
+            if (row < 32) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sw[row * RS + 4 * p + e] = pc[k][e];
+            }
+        }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+    };
+    // the activations through buffers that end with this workgroup's tiles:
+    // blocks past the slice are out of range and read nothing
+    const int a_bytes = TT * nb * 8 * 1024, x_bytes = TT * nb * 32 * (int)sizeof(float);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t*>(L.qs) + (size_t)t32 * nb * 8 * 1024, 0, a_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(L.xd) + (size_t)t32 * nb * 32, 0, x_bytes, 0x00020000);
+    i32x4 av[TT][8];
+    float xd[TT];
+    auto load_a = [&](int j, int k) __attribute__((always_inline)) {  // slabs 2 k, 2 k + 1 of every tile
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+            for (int s = 2 * k; s < 2 * k + 2; ++s)
+                av[tt][s] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                          ra, j < cnt ? ((tt * nb + b0 + j) * 8 + s) * 1024 + lane * 16 : a_bytes, 0, 0));
+    };
+    auto load_x = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+            xd[tt] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                rx, j < cnt ? ((tt * nb + b0 + j) * 32 + c) * (int)sizeof(float) : x_bytes, 0, 0));
+    };
+    f32x16 sum[TT];
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sum[tt][i] = 0.0f;
+    const f32x16 z = {};
+    load_w(0);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) load_a(0, k);
+    load_x(0);
+    for (int it = 0; it < cnt; ++it) {
+        store_w();
+        load_w(it + 1);
+        const int mis = (mis0 + c * row_b + (b0 + it) * WB) & 3;  // this lane's row starts mis bytes into its LDS row
+        auto at = [&](int byte) __attribute__((always_inline)) {  // 4 bytes at an even offset
+            const int o = mis + byte;
+            const uint32_t* row = sw + c * RS;
+            return __builtin_amdgcn_alignbit(row[(o >> 2) + 1], row[o >> 2], (o & 2) * 8);
+        };
+        auto at16 = [&](int byte) __attribute__((always_inline)) {
+            return u32x4{at(byte), at(byte + 4), at(byte + 8), at(byte + 12)};
+        };
+        __builtin_amdgcn_sched_barrier(0);  // (the loads would sink to their use)
+        BlockScale bsc;
+        i32x16 hi[TT], lo[TT];
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) hi[tt] = lo[tt] = i32x16{};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            u32x4 w[2][2];  // [slab of the pair][hi / lo]
+            RawBlock<14> r;  // (ql runs 64 h + 32 a + 16 g, qh run 32 h + 16 g, src/kernels.rs:135-147)
+            const int h = k >> 1;
+            r.sc = at16(192);
+            r.ql[0] = at16(64 * h + 16 * g);
+            r.ql[1] = at16(64 * h + 32 + 16 * g);
+            r.qh = at16(128 + 32 * h + 16 * g);
+            r.d = at(208) & 0xFFFFu;
+            form_pair(r, k, lane, w, bsc);
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int tt = 0; tt < TT; ++tt) {
+                    hi[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[tt][2 * k + s], __builtin_bit_cast(i32x4, w[s][0]),
+                                                                   hi[tt], 0, 0, 0);
+                    lo[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[tt][2 * k + s], __builtin_bit_cast(i32x4, w[s][1]),
+                                                                   lo[tt], 0, 0, 0);
+                }
+            load_a(it + 1, k);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) {
+            const float xa = g == 0 ? xd[tt] : 0.0f;
+            const f32x16 dd = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, g == 0 ? bsc.wd : 0.0f, z, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int v = (hi[tt][i] << SHIFT) + lo[tt][i];
+                sum[tt][i] = __builtin_fmaf(dd[i], (float)v, sum[tt][i]);
+            }
+        }
+        load_x(it + 1);
+    }
+    __syncthreads();  // the blocks' LDS becomes the slices' sums
+    finish_slices<TT>(a, sum, *reinterpret_cast<float(*)[8][16][64]>(s_mem), wave, lane, t32 * 32, rt);
 }
 
 // Gemma's post-attention RMSNorm before the residual add (forward.rs:346-350):
@@ -1185,12 +1318,13 @@ size_t qmm0_workspace_bytes(int n, int cols) {
 // work they repeat per 64 activation rows counts (forming the weight
 // operands, for the 32-value types shifting them out of LDS).  Calls, us,
 // walk / slices, 4096 x 4096 unless noted:
-//   Q4_K  n 20 20.4 / 12.0, 60 21.0 / 15.2, 120 21.2 / 15.9, 190 22.2 / 25.1,
-//         256 22.6 / 25.9; 2048 x 2048 n 256 14.8 / 11.4, 512 16.4 / 18.4
+//   Q4_K  n 20 20.3 / 11.7, 64 20.8 / 13.9, 128 21.0 / 14.9, 190 22.2 / 25.1,
+//         256 22.6 / 24.4, 512 40.8 / 41.9; 2048 x 2048 n 256 14.9 / 11.1, 512
+//         16.5 / 16.5
 //   Q4_0  n 20 28.5 / 12.1, 60 29.0 / 17.4, 120 29.3 / 18.3, 256 30.3 / 32.1
 // Q6_K always takes slices: its operands cost more to form than to share
-// through LDS (n 60 34.5 / 17.3, 256 35.7 / 30.9; 2048 x 4096, 2553 rows with
-// the norm, 176 / 134).
+// through LDS (n 60 34.5 / 15.3, 256 35.7 / 29.8; 2048 x 4096, 2553 rows with
+// the norm, 176 / 130).
 static bool use_slices(const QmmArgs& a) {
     return a.wtype == 14 || (a.rows + 31) / 32 * ((a.n + 63) / 64) <= 256;
 }
@@ -1205,9 +1339,9 @@ static void launch_slices(const QmmArgs& a, hipStream_t st) {
     const dim3 grid(n_rt * (one ? 1u : (unsigned)((a.n + 63) / 64)));
     if constexpr (WT == 12 || WT == 14) {
         if (one)
-            hipLaunchKernelGGL((qmm_slice_kernel<WT, 1>), grid, dim3(512), 0, st, a);
+            hipLaunchKernelGGL(WT == 12 ? qmm_slice_kernel<1> : qmm6_slice_kernel<1>, grid, dim3(512), 0, st, a);
         else
-            hipLaunchKernelGGL((qmm_slice_kernel<WT, 2>), grid, dim3(512), 0, st, a);
+            hipLaunchKernelGGL(WT == 12 ? qmm_slice_kernel<2> : qmm6_slice_kernel<2>, grid, dim3(512), 0, st, a);
     } else {
         if (one)
             hipLaunchKernelGGL((qmm0_slice_kernel<WT, 1>), grid, dim3(512), 0, st, a);
