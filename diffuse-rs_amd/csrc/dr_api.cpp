@@ -986,6 +986,13 @@ static void wtype_block(int wtype, size_t& qk, size_t& bytes) {
     }
 }
 
+// sizes (none of them 0) that the kernels' index arithmetic holds
+static bool qmm_size_ok(size_t qk, size_t rows, size_t cols, size_t n) {
+    return rows > 0 && n > 0 && cols > 0 && cols % qk == 0 && rows <= (size_t)INT32_MAX &&
+           cols <= (size_t)INT32_MAX / 2 && n <= (size_t)INT32_MAX / 2 &&
+           (size_t)dr::qmm_rows_padded((int)n) * (cols / qk) * (qk == 32 ? 64 : 1) <= (size_t)INT32_MAX;
+}
+
 static int qmatmul_impl(dr_ctx* ctx, int wtype, const void* w, size_t rows, size_t cols, const float* act,
                         size_t n, float* out, const float* residual, const float* norm_w, float eps,
                         const char* who) {
@@ -1004,9 +1011,7 @@ static int qmatmul_impl(dr_ctx* ctx, int wtype, const void* w, size_t rows, size
         return fail(DR_ERR_INVALID, "%s: Q4_K blocks must start 16-byte aligned (16-byte loads)", who);
     if (((uintptr_t)w & 1) || ((uintptr_t)act & 15))
         return fail(DR_ERR_INVALID, "%s: weight blocks must start 2-byte aligned and act 16-byte aligned", who);
-    const size_t nb = cols / qk;
-    if (rows > (size_t)INT32_MAX || cols > (size_t)INT32_MAX / 2 || n > (size_t)INT32_MAX / 2 ||
-        (size_t)dr::qmm_rows_padded((int)n) * nb * (qk == 32 ? 64 : 1) > (size_t)INT32_MAX)
+    if (!qmm_size_ok(qk, rows, cols, n))
         return fail(DR_ERR_INVALID, "%s: %zu x %zu x %zu too large", who, n, rows, cols);
     DR_CHECK(use_device(ctx));
     const size_t ws = qk == 32 ? dr::qmm0_workspace_bytes((int)n, (int)cols) : dr::qmm_workspace_bytes((int)n, (int)cols);
@@ -1761,6 +1766,21 @@ int dr_attention(float* out, size_t out_len, const float* q, size_t q_len, const
 }
 
 long dr_debug_alloc_count(void) { return g_allocs.load(std::memory_order_relaxed); }
+
+int dr_debug_qmm_plan(int wtype, size_t rows, size_t cols, size_t n, int* slices, size_t* max_offset,
+                      size_t* workgroups) {
+    size_t qk, bb;
+    wtype_block(wtype, qk, bb);
+    if (!qk) return fail(DR_ERR_UNSUPPORTED, "dr_debug_qmm_plan: weight type %d not built", wtype);
+    if (!slices || !max_offset || !workgroups || !qmm_size_ok(qk, rows, cols, n))
+        return fail(DR_ERR_INVALID, "dr_debug_qmm_plan: %zu x %zu x %zu", n, rows, cols);
+    const bool sl = dr::qmm_slices(wtype, (int)rows, (int)cols, (int)n);
+    *slices = sl ? 1 : 0;
+    *max_offset = sl ? dr::qmm_slice_offset(wtype, (int)cols, (int)n) : 0;
+    *workgroups = sl ? dr::qmm_slice_workgroups((int)rows, (int)n)
+                     : (rows + 31) / 32 * ((size_t)dr::qmm_rows_padded((int)n) / 128);
+    return DR_OK;
+}
 
 int dr_debug_ring_tiles(size_t head_dim, size_t nk, size_t cap, long long window, long long qmin,
                         long long qmax, size_t n_split, int* min_tile, int* max_tile, int* partition_ok) {

@@ -387,6 +387,11 @@ hipError_t launch_epilogue(const EpiArgs& a, hipStream_t st);
 hipError_t launch_split_active(const SplitArgs& a, hipStream_t st);
 size_t qmm_workspace_bytes(int n, int cols);
 size_t qmm0_workspace_bytes(int n, int cols);  // the legacy block types
+// dr_qmatmul's kernels: the slices of the blocks (true) or the walk over all
+// of them; the slices' workgroups and the largest 32-bit offset they form.
+bool qmm_slices(int wtype, int rows, int cols, int n);
+size_t qmm_slice_workgroups(int rows, int n);
+size_t qmm_slice_offset(int wtype, int cols, int n);
 hipError_t launch_qmatmul(const QmmArgs& a, hipStream_t st);
 // quantize_row_q8_0 into the reference's BlockQ8_0 layout (34 bytes each)
 hipError_t launch_quantize_q80(const float* act, int n, int cols, void* out, hipStream_t st);

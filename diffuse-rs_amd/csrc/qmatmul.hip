@@ -237,7 +237,6 @@ __global__ __launch_bounds__(512) void q8k_quantize_tiles_kernel(const float* __
 // slab s of row c; accumulator slot i of that lane is output (t = 8 (i / 4) +
 // 4 g + i % 4, r = c).
 //
-// (This kernel runs Q4_K only; Q6_K always takes qmm6_slice_kernel below.)
 // Weight operand of a Q4_K block: slab s = sub-block s.  sc_s = 8 sh + sl with
 // sh, sl <= 7, so sh * q and sl * q (q <= 15) are bytes and a 16-bit packed
 // multiply scales two nibble bytes at once without carries; the two parts
@@ -270,6 +269,16 @@ struct RawBlock<14> {
 __device__ __forceinline__ void load_raw(const uint8_t* blk, int c, int g, RawBlock<12>& r) {
     r.h = gld<u32x4>(blk);
     r.q = gld<u32x4>(blk + 16 + 32 * c + 16 * g);
+}
+// slabs 2 c, 2 c + 1 of a Q6_K block: half c / 2, quarters 2 (c % 2), + 1
+// (src/kernels.rs:135-147): ql runs 64 h + 32 a + 16 g, qh run 32 h + 16 g
+__device__ __forceinline__ void load_raw(const uint8_t* blk, int c, int g, RawBlock<14>& r) {
+    const int h = c >> 1;
+    r.sc = gld16_a2(blk + 192);
+    r.ql[0] = gld16_a2(blk + 64 * h + 16 * g);
+    r.ql[1] = gld16_a2(blk + 64 * h + 32 + 16 * g);
+    r.qh = gld16_a2(blk + 128 + 32 * h + 16 * g);
+    r.d = gld<uint16_t>(blk + 208);
 }
 // What the combine of a block needs besides the MFMA results.
 struct BlockScale {
@@ -377,9 +386,11 @@ __device__ __forceinline__ void store_tile(const QmmArgs& a, int t0, int g, int 
     }
 }
 
+template <int WT>
 __global__ __launch_bounds__(512) void qmm_kernel(const QmmArgs a) {
-    constexpr int WB = Q4K_BYTES;
-    constexpr int SHIFT = 3;
+    constexpr bool Q4 = WT == 12;
+    constexpr int WB = Q4 ? Q4K_BYTES : Q6K_BYTES;
+    constexpr int SHIFT = Q4 ? 3 : 6;
     // B operands [buffer][half][slab][hi / lo][lane] (64 KB); after the loop
     // the first 16 KB carry half 1's partial sums [tile][slot][lane]
     __shared__ u32x4 s_b[2][2][8][2][64];
@@ -422,7 +433,7 @@ __global__ __launch_bounds__(512) void qmm_kernel(const QmmArgs a) {
         bf16x8 bm;
     };
     Stage S[2];
-    RawBlock<12> R[2];
+    RawBlock<WT> R[2];
     BlockScale bsc;
     const int blast = kb0 + (kcnt > 0 ? kcnt - 1 : 0);
     auto load_stage = [&](int b, Stage& st) __attribute__((always_inline)) {
@@ -430,7 +441,7 @@ __global__ __launch_bounds__(512) void qmm_kernel(const QmmArgs a) {
 #pragma unroll
         for (int s = 0; s < 8; ++s) st.av[s] = gld<i32x4>(abase + ((size_t)b * 8 + s) * 1024);
         st.xd = gld<float>(xbase + (size_t)b * 32);
-        st.bm = gld<bf16x8>(mbase + (size_t)b * 64 * 8);
+        if constexpr (Q4) st.bm = gld<bf16x8>(mbase + (size_t)b * 64 * 8);
     };
     // The combine of a block runs in the next iteration, under that block's
     // MFMA chains: the products of the previous block wait in registers.
@@ -444,10 +455,10 @@ __global__ __launch_bounds__(512) void qmm_kernel(const QmmArgs a) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             sum[i] = __builtin_fmaf(pr.dd[i], (float)pr.acc[i], sum[i]);
-            sum[i] = __builtin_fmaf(-pr.dm[i], pr.mins[i], sum[i]);
+            if constexpr (Q4) sum[i] = __builtin_fmaf(-pr.dm[i], pr.mins[i], sum[i]);
         }
     };
-    auto body = [&](int it, Stage& cur, Stage& nxt, RawBlock<12>& rprep, RawBlock<12>& rload, int buf)
+    auto body = [&](int it, Stage& cur, Stage& nxt, RawBlock<WT>& rprep, RawBlock<WT>& rload, int buf)
         __attribute__((always_inline)) {
         if (it < kcnt) {
             load_stage(min(kb0 + it + 1, blast), nxt);
@@ -472,14 +483,14 @@ __global__ __launch_bounds__(512) void qmm_kernel(const QmmArgs a) {
                     cur.av[s], __builtin_bit_cast(i32x4, bsrc[(s * 2 + 1) * 64]), acc, 0, 0, 0);
             np.acc = acc;
             np.mins = f32x16{};
-            np.mins = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.bm, bsc.mn, np.mins, 0, 0, 0);
+            if constexpr (Q4) np.mins = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.bm, bsc.mn, np.mins, 0, 0, 0);
             // the block scales d_x d_w (and d_x dmin_w) of every slot, each one
             // f32 product, on a K = 2 f32 MFMA with the second K row zero
             const float xa = g == 0 ? cur.xd : 0.0f;
             const f32x16 z = {};
             np.dd = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, g == 0 ? bsc.wd : 0.0f, z, 0, 0, 0);
             np.dm = f32x16{};
-            np.dm = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, g == 0 ? bsc.wdmin : 0.0f, z, 0, 0, 0);
+            if constexpr (Q4) np.dm = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, g == 0 ? bsc.wdmin : 0.0f, z, 0, 0, 0);
             // ---- under the second chain: the next block's B operands into the
             // other buffer (past the last block: a repeat nobody reads)
             prep(rprep, c, lane, &s_b[buf ^ 1][kh][0][0][0], bsc);
@@ -489,7 +500,7 @@ __global__ __launch_bounds__(512) void qmm_kernel(const QmmArgs a) {
         lds_barrier();
     };
     if (kcnt > 0) {
-        RawBlock<12> raw0;
+        RawBlock<WT> raw0;
         load_raw(wrow + (size_t)kb0 * WB, c, g, raw0);
         load_stage(kb0, S[0]);
         load_raw(wrow + (size_t)min(kb0 + 1, blast) * WB, c, g, R[1]);
@@ -782,7 +793,7 @@ __global__ __launch_bounds__(512) void qmm0_kernel(const QmmArgs a) {
 
 // ---------------------------------------------------------------------------
 // Slices of the blocks: calls whose grid would leave CUs idle (an MoE
-// expert's rows, short canvases), and all of Q6_K; see use_slices.  The
+// expert's rows, short canvases), and Q6_K; see qmm_slices.  The
 // kernels that walk every block take one memory round trip after the other
 // (a block or a group of blocks, then a barrier).  Here the 8 waves of a
 // workgroup take an eighth of the blocks each, for 32 weight rows and TT tiles
@@ -1311,6 +1322,33 @@ size_t qmm0_workspace_bytes(int n, int cols) {
     return n_pad * cols + n_pad * nb * sizeof(float);
 }
 
+// The largest byte offset that a slice kernel forms into the weights or the
+// activations (its buffers take 32-bit offsets; one block past a slice is
+// formed and not loaded).  Q4_K: its addresses are 64-bit.
+template <int WT>
+static size_t legacy_slice_offset(size_t nb) {
+    using G = SliceGeom<WT>;
+    const size_t w_rows = (G::NL * 64 - 1) / G::NP + 1;  // (rows past 32 are formed and not loaded)
+    return w_rows * nb * G::BB + G::CB * G::BB + 16 * G::NP + 3;
+}
+size_t qmm_slice_offset(int wtype, int cols, int n) {
+    const size_t nb = (size_t)cols / (wtype == 14 ? QK : 32);
+    switch (wtype) {
+        case 14: {
+            const size_t acts = ((n <= 32 ? 1 : 2) * nb + 1) * 8 * 1024;  // tiles of a workgroup, 8 slabs of 1 KB a block
+            const size_t weights = 32 * nb * Q6K_BYTES + Q6K_BYTES + 16 * 16 + 3;
+            return std::max(acts, weights);
+        }
+        case 2: return legacy_slice_offset<2>(nb);
+        case 6: return legacy_slice_offset<6>(nb);
+        case 8: return legacy_slice_offset<8>(nb);
+        default: return 0;
+    }
+}
+size_t qmm_slice_workgroups(int rows, int n) {
+    return (size_t)((rows + 31) / 32) * (size_t)(n <= 32 ? 1 : (n + 63) / 64);
+}
+
 // The slice kernels (an eighth of the blocks per wave, 32 weight rows x 32 or
 // 64 activation rows per workgroup) or the ones that walk all blocks of 32 x
 // 128.  A walk costs a round trip per block or group of blocks whatever the
@@ -1325,18 +1363,23 @@ size_t qmm0_workspace_bytes(int n, int cols) {
 // Q6_K always takes slices: its operands cost more to form than to share
 // through LDS (n 60 34.5 / 15.3, 256 35.7 / 29.8; 2048 x 4096, 2553 rows with
 // the norm, 176 / 130).
-static bool use_slices(const QmmArgs& a) {
-    return a.wtype == 14 || (a.rows + 31) / 32 * ((a.n + 63) / 64) <= 256;
+// Rows too long for the slices' 32-bit offsets (Q6_K from 2^25 columns on) and
+// grids past a launch's 2^32 threads, which the walk's larger tiles reach at
+// twice the size, walk.
+bool qmm_slices(int wtype, int rows, int cols, int n) {
+    const size_t wgs = qmm_slice_workgroups(rows, n);
+    if (qmm_slice_offset(wtype, cols, n) > INT32_MAX || wgs * 512 > UINT32_MAX) return false;
+    return wtype == 14 || wgs <= 256;
 }
+static bool use_slices(const QmmArgs& a) { return qmm_slices(a.wtype, a.rows, a.cols, a.n); }
 // Activation tiles that the matmul reads.
 static int quantized_tiles(const QmmArgs& a) {
     return !use_slices(a) ? a.n_pad / 32 : (a.n <= 32 ? 1 : (a.n + 63) / 64 * 2);
 }
 template <int WT>
 static void launch_slices(const QmmArgs& a, hipStream_t st) {
-    const unsigned n_rt = (unsigned)((a.rows + 31) / 32);
     const bool one = a.n <= 32;
-    const dim3 grid(n_rt * (one ? 1u : (unsigned)((a.n + 63) / 64)));
+    const dim3 grid((unsigned)qmm_slice_workgroups(a.rows, a.n));
     if constexpr (WT == 12 || WT == 14) {
         if (one)
             hipLaunchKernelGGL(WT == 12 ? qmm_slice_kernel<1> : qmm6_slice_kernel<1>, grid, dim3(512), 0, st, a);
@@ -1399,13 +1442,13 @@ hipError_t launch_qmatmul(const QmmArgs& a, hipStream_t st) {
         b.residual = nullptr;
         b.out = a.norm_tmp;
     }
-    if (a.wtype != 12 && a.wtype != 14) return hipErrorInvalidValue;
-    if (a.wtype == 14)
-        launch_slices<14>(b, st);
-    else if (use_slices(a))
-        launch_slices<12>(b, st);
-    else
-        hipLaunchKernelGGL(qmm_kernel, dim3(nwg), dim3(512), 0, st, b);
+    switch (a.wtype * 2 + (use_slices(a) ? 1 : 0)) {
+        case 24: hipLaunchKernelGGL(qmm_kernel<12>, dim3(nwg), dim3(512), 0, st, b); break;
+        case 25: launch_slices<12>(b, st); break;
+        case 28: hipLaunchKernelGGL(qmm_kernel<14>, dim3(nwg), dim3(512), 0, st, b); break;
+        case 29: launch_slices<14>(b, st); break;
+        default: return hipErrorInvalidValue;
+    }
     e = hipGetLastError();
     if (e != hipSuccess || !a.norm_w) return e;
     hipLaunchKernelGGL(post_norm_kernel, dim3((unsigned)a.n), dim3(256), 0, st, a.norm_tmp, a.out, a.norm_w,

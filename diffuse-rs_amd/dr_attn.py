@@ -178,6 +178,7 @@ _SIGS = {
     "dr_debug_alloc_count": (ctypes.c_long, []),
     "dr_debug_ring_tiles": (_I, [_SZ, _SZ, _SZ, ctypes.c_longlong, ctypes.c_longlong, ctypes.c_longlong, _SZ,
                                  ctypes.POINTER(_I), ctypes.POINTER(_I), ctypes.POINTER(_I)]),
+    "dr_debug_qmm_plan": (_I, [_I, _SZ, _SZ, _SZ, ctypes.POINTER(_I), c_size_p, c_size_p]),
 }
 
 
@@ -655,6 +656,14 @@ def ring_tiles(head_dim: int, nk: int, cap: int, window: Optional[int], qmin: in
     _check(load().dr_debug_ring_tiles(head_dim, nk, cap, -1 if window is None else window, qmin, qmax,
                                       n_split, ctypes.byref(lo), ctypes.byref(hi), ctypes.byref(ok)))
     return lo.value, hi.value, bool(ok.value)
+
+
+def qmm_plan(wtype: int, rows: int, cols: int, n: int) -> tuple:
+    """(slices, largest 32-bit offset, workgroups) of dr_qmatmul's kernel for
+    these sizes (dr_debug_qmm_plan); host-only."""
+    sl, off, wgs = ctypes.c_int(), ctypes.c_size_t(), ctypes.c_size_t()
+    _check(load().dr_debug_qmm_plan(wtype, rows, cols, n, ctypes.byref(sl), ctypes.byref(off), ctypes.byref(wgs)))
+    return bool(sl.value), off.value, wgs.value
 
 
 def qmatmul_post_norm(ctx: Context, wtype: int, w, rows: int, cols: int, act, n: int, out, norm_w,

@@ -151,6 +151,41 @@ def test_ring_kernel_dma_stays_inside_the_cache_plane(lib):
         dr.ring_tiles(64, 32, 64, None, 0, 0, 1)  # no stream kernel at hd 64
 
 
+@pytest.mark.parametrize("wtype,qk,bb", [(12, 256, 144), (14, 256, 210), (2, 32, 18), (6, 32, 22), (8, 32, 34)])
+def test_qmatmul_slice_offsets_fit_32_bits(lib, wtype, qk, bb):
+    """The slice kernels address the 32 weight rows and the one or two tiles
+    of activations of a workgroup with 32-bit offsets: a size whose offsets do
+    not fit takes the walking kernel (64-bit addresses), over every row length
+    that dr_qmatmul accepts.  So does a grid past a launch's 2^32 threads that
+    the walk's larger tiles still fit."""
+    took = set()
+    for bits in range(31):
+        for cols in {(1 << bits) // qk * qk, ((1 << bits) + qk) // qk * qk, (3 << bits) // 2 // qk * qk}:
+            for n in (1, 32, 33, 64, 129):
+                try:
+                    slices, off, _ = dr.qmm_plan(wtype, 32, cols, n)
+                except dr.DrError:
+                    continue  # refused by dr_qmatmul too
+                took.add(slices)
+                if not slices:
+                    continue
+                nb, tiles = cols // qk, 1 if n <= 32 else 2
+                assert off < 2 ** 31, (cols, n)
+                if wtype != 12:  # (Q4_K: 64-bit addresses)
+                    assert off >= 32 * nb * bb, (cols, n)
+                if wtype == 14:
+                    assert off >= tiles * nb * 8 * 1024, (cols, n)
+    assert True in took
+    if wtype == 14:  # 2 tiles x 2^18 blocks x 8 KB are 2^32 bytes: as 32 bits, none
+        assert not dr.qmm_plan(14, 32, 1 << 26, 33)[0] and not dr.qmm_plan(14, 1, 1 << 27, 1)[0]
+        assert dr.qmm_plan(14, 32, 1 << 24, 33)[0]
+    for rows in (1 << 17, 1 << 18, 151936):
+        for n in (65600, 131200):
+            _, _, wgs = dr.qmm_plan(wtype, rows, 256, n)
+            walk = (rows + 31) // 32 * ((n + 127) // 128)
+            assert wgs * 512 < 2 ** 32 or walk * 512 >= 2 ** 32, (rows, n, wgs)
+
+
 def test_alloc_counter_counts_no_device_calls(lib):
     """The allocation counter is host-side state: readable without a GPU and
     unchanged by calls that fail before allocating."""

@@ -43,3 +43,32 @@ def test_qmatmul_slices_vs_oracle(dev, wtype, rows, blocks, n, skew):
     out = dev.put(res.reshape(-1))
     dr.qmatmul(dev.ctx, wtype, buf.data_ptr() + skew, rows, cols, dev.put(x), n, out, out)
     _check(dev.get(out).reshape(n, rows), want, tol, f"wtype {wtype} {rows} x {cols}, {n} rows, skew {skew}")
+
+
+def test_q6k_rows_past_32_bit_offsets(dev):
+    """Q6_K over 2^26 columns and 33 activation rows: two tiles of Q8_K
+    activations are 2^32 bytes, past the slices' 32-bit offsets.  All but a few
+    blocks of the activations are zero and add nothing, so the oracle runs on
+    those blocks alone."""
+    t, rows, n, nb = dev.t, 2, 33, 1 << 18
+    at = [0, 1, 4095, (1 << 17) - 1, 1 << 17, (1 << 17) + 1, nb - 2, nb - 1]
+    rng = np.random.default_rng(26)
+    cols = 256 * len(at)
+    w, x = kquant_weights(rng, orc.WTYPE_Q6K, rows, cols), kquant_acts(rng, n, cols)
+    res = rng.standard_normal((n, rows)).astype(np.float32)
+    want = orc.qmatmul(orc.WTYPE_Q6K, w, rows, cols, x, n, res).reshape(n, rows)
+    tol = kquant_bound(orc, orc.WTYPE_Q6K, w, rows, cols, x, n, res)
+    ctx = dr.Context(0)  # (its workspace of 10 GB goes with it)
+    ctx.set_stream(dev.stream.cuda_stream)
+    with t.cuda.stream(dev.stream):
+        wd = t.zeros((rows, nb, 210), dtype=t.uint8, device="cuda")
+        xd = t.zeros((n, nb, 256), dtype=t.float32, device="cuda")
+        wd[:, at] = t.from_numpy(w.reshape(rows, len(at), 210)).cuda()
+        xd[:, at] = t.from_numpy(x.reshape(n, len(at), 256)).cuda()
+    out = dev.put(res.reshape(-1))
+    dr.qmatmul(ctx, orc.WTYPE_Q6K, wd, rows, nb * 256, xd, n, out, out)
+    got = dev.get(out).reshape(n, rows)
+    ctx.close()
+    del wd, xd
+    t.cuda.empty_cache()
+    _check(got, want, tol, f"Q6_K {rows} x {nb * 256}, {n} rows")
