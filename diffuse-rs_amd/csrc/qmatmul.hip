@@ -286,9 +286,10 @@ struct BlockScale {
     bf16x8 mn;  // Q4_K: the eight 6-bit mins (B operand of the min MFMA)
 };
 
-// Scales of a block, and the B operands of its slabs 2 c and 2 c + 1 (w[slab][hi
-// / lo]); prep writes them to LDS (dst[slab][hi / lo][lane]).
-__device__ __forceinline__ void form_pair(const RawBlock<12>& r, int c, int lane, u32x4 (&w)[2][2], BlockScale& o) {
+// Scales of a block, and the B operands of its slabs 2 c and 2 c + 1, each
+// slab handed to put(slab of the pair, hi, lo) as it is formed.
+template <typename Put>
+__device__ __forceinline__ void form_pair(const RawBlock<12>& r, int c, int lane, BlockScale& o, Put put) {
     const u32x4 h = r.h;
     o.wd = f16_to_f32(h.x & 0xFFFF);
     o.wdmin = f16_to_f32(h.x >> 16);
@@ -314,12 +315,12 @@ __device__ __forceinline__ void form_pair(const RawBlock<12>& r, int c, int lane
             vh[k] = pk_mul_u16(nib, fh);
             vl[k] = pk_mul_u16(nib, fl);
         }
-        w[hn][0] = vh;
-        w[hn][1] = vl;
+        put(hn, vh, vl);
     }
 }
 
-__device__ __forceinline__ void form_pair(const RawBlock<14>& r, int c, int lane, u32x4 (&w)[2][2], BlockScale& o) {
+template <typename Put>
+__device__ __forceinline__ void form_pair(const RawBlock<14>& r, int c, int lane, BlockScale& o, Put put) {
     o.wd = f16_to_f32(r.d);
     o.wdmin = 0.0f;
     const int g = lane >> 5;
@@ -344,19 +345,28 @@ __device__ __forceinline__ void form_pair(const RawBlock<14>& r, int c, int lane
             vh[k] = pack_lo_bytes(pk_ashr_i16(w01, 6), pk_ashr_i16(w23, 6));
             vl[k] = pack_lo_bytes(w01 & 0x003F003Fu, w23 & 0x003F003Fu);
         }
-        w[k2][0] = vh;
-        w[k2][1] = vl;
+        put(k2, vh, vl);
     }
 }
 
+// The same into LDS (dst[slab][hi / lo][lane]).  A slab is written as soon as
+// it is formed: with all four operands formed first the kernel takes 0.5-2 %
+// longer (4096 x 4096, 512 rows: 40.8 -> 41.7 us).
 template <int WT>
 __device__ __forceinline__ void prep(const RawBlock<WT>& r, int c, int lane, u32x4* dst, BlockScale& o) {
-    u32x4 w[2][2];
-    form_pair(r, c, lane, w, o);
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int p = 0; p < 2; ++p) dst[((2 * c + s) * 2 + p) * 64 + lane] = w[s][p];
+    form_pair(r, c, lane, o, [&](int s, u32x4 hi, u32x4 lo) __attribute__((always_inline)) {
+        dst[((2 * c + s) * 2 + 0) * 64 + lane] = hi;
+        dst[((2 * c + s) * 2 + 1) * 64 + lane] = lo;
+    });
+}
+
+// The same in registers (w[slab of the pair][hi / lo]).
+template <int WT>
+__device__ __forceinline__ void form_pair(const RawBlock<WT>& r, int c, int lane, u32x4 (&w)[2][2], BlockScale& o) {
+    form_pair(r, c, lane, o, [&](int s, u32x4 hi, u32x4 lo) __attribute__((always_inline)) {
+        w[s][0] = hi;
+        w[s][1] = lo;
+    });
 }
 
 // The residual of a lane's 16 outputs (activation rows t0 + 8 (i / 4) + 4 g
