@@ -186,6 +186,15 @@ def test_qmatmul_slice_offsets_fit_32_bits(lib, wtype, qk, bb):
             assert wgs * 512 < 2 ** 32 or walk * 512 >= 2 ** 32, (rows, n, wgs)
 
 
+def test_qmatmul_q6k_few_blocks_walk_past_one_round(lib):
+    """Q6_K grids past one workgroup per CU: rows of 1, 2, 6 or 10 blocks take
+    the walking kernel (measured faster there), all others the slices; up to
+    one per CU all take the slices."""
+    for nb in range(1, 41):
+        assert dr.qmm_plan(14, 4096, 256 * nb, 128)[0]  # 256 workgroups
+        assert dr.qmm_plan(14, 4096, 256 * nb, 129)[0] == (nb not in (1, 2, 6, 10)), nb
+
+
 def test_alloc_counter_counts_no_device_calls(lib):
     """The allocation counter is host-side state: readable without a GPU and
     unchanged by calls that fail before allocating."""

@@ -26,7 +26,7 @@ TYPES = [orc.WTYPE_Q4K, orc.WTYPE_Q6K, orc.WTYPE_Q4_0, orc.WTYPE_Q5_0, orc.WTYPE
 @pytest.mark.parametrize("wtype", TYPES)
 @pytest.mark.parametrize("rows,blocks,n,skew", [
     (1, 1, 1, 0), (31, 3, 32, 2), (33, 8, 33, 0), (65, 9, 64, 2), (40, 17, 65, 0), (70, 40, 129, 2),
-    (32 * 256 + 1, 2, 64, 0),  # 257 workgroups: the walking kernels (Q6_K: slices)
+    (32 * 256 + 1, 2, 64, 0),  # 257 workgroups: the walking kernels
     (32 * 64 + 1, 5, 257, 0),
 ])
 def test_qmatmul_slices_vs_oracle(dev, wtype, rows, blocks, n, skew):
