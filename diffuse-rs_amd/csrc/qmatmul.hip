@@ -1370,6 +1370,12 @@ size_t qmm_slice_workgroups(int rows, int n) {
 //         256 22.6 / 24.4, 512 40.8 / 41.9; 2048 x 2048 n 256 14.9 / 11.1, 512
 //         16.5 / 16.5
 //   Q4_0  n 20 28.5 / 12.1, 60 29.0 / 17.4, 120 29.3 / 18.3, 256 30.3 / 32.1
+//   1024 x 2048  Q5_0 n 32 19.0 / 9.7, 64 19.2 / 12.5; Q8_0 n 32 17.4 / 8.3, 64 17.5 / 11.1
+// Q4_0 and Q5_0 rows of 2 to 8 blocks give a wave one block, and shifting it
+// out of LDS for two tiles takes longer than the walk (2048 rows of 256
+// columns, n 96: Q4_0 8.1 / 8.8, Q5_0 8.1 / 9.0; 32 columns 7.4 / 6.9, 7.6 /
+// 7.0; 288 9.3 / 8.4, 9.7 / 8.4; n 32, one tile, 256 columns 7.8 / 7.1, 8.0 /
+// 7.4; Q8_0 n 96 7.9 / 7.6).
 // Q6_K takes slices past that too: its operands cost more to form than to
 // share through LDS (n 60 34.5 / 15.3, 256 35.7 / 29.8; 2048 x 4096, 2553 rows
 // with the norm, 176 / 130).  Not for rows of 1, 2, 6 and 10 blocks, which
@@ -1377,14 +1383,14 @@ size_t qmm_slice_workgroups(int rows, int n) {
 // halves are even (4096 weight rows, 1024 activation rows: 256 columns 25 / 38,
 // 512 30 / 39, 768 51 / 41, 1024 53 / 44, 1280 56 / 54, 1536 53 / 56, 1792 75
 // / 58, 2048 74 / 60, 2304 89 / 69, 2560 75 / 83, 2816 105 / 86, 4608 125 /
-// 115, and 1.15 or more at every other length up to 40 blocks).
+// 115, and 1.07 or more at every other length up to 40 blocks).
 // Rows too long for the slices' 32-bit offsets (Q6_K from 2^25 columns on) and
 // grids past a launch's 2^32 threads, which the walk's larger tiles reach at
 // twice the size, walk.
 bool qmm_slices(int wtype, int rows, int cols, int n) {
     const size_t wgs = qmm_slice_workgroups(rows, n);
     if (qmm_slice_offset(wtype, cols, n) > INT32_MAX || wgs * 512 > UINT32_MAX) return false;
-    if (wgs <= 256) return true;
+    if (wgs <= 256) return !((wtype == 2 || wtype == 6) && n > 32 && cols > 32 && cols <= 8 * 32);
     const int nb = cols / QK;
     return wtype == 14 && nb != 1 && !(nb % 4 == 2 && nb <= 10);
 }

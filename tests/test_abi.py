@@ -195,6 +195,15 @@ def test_qmatmul_q6k_few_blocks_walk_past_one_round(lib):
         assert dr.qmm_plan(14, 4096, 256 * nb, 129)[0] == (nb not in (1, 2, 6, 10)), nb
 
 
+@pytest.mark.parametrize("wtype", [2, 6, 8])
+def test_qmatmul_short_legacy_rows_walk_with_two_tiles(lib, wtype):
+    """Q4_0 and Q5_0 rows of 2 to 8 blocks and more than 32 activation rows
+    take the walking kernel (measured faster there); Q8_0 the slices."""
+    for cols in range(32, 544, 32):
+        assert dr.qmm_plan(wtype, 1024, cols, 32)[0]
+        assert dr.qmm_plan(wtype, 1024, cols, 33)[0] == (wtype == 8 or cols == 32 or cols > 256), cols
+
+
 def test_alloc_counter_counts_no_device_calls(lib):
     """The allocation counter is host-side state: readable without a GPU and
     unchanged by calls that fail before allocating."""
