@@ -1383,7 +1383,10 @@ size_t qmm_slice_workgroups(int rows, int n) {
 // halves are even (4096 weight rows, 1024 activation rows: 256 columns 25 / 38,
 // 512 30 / 39, 768 51 / 41, 1024 53 / 44, 1280 56 / 54, 1536 53 / 56, 1792 75
 // / 58, 2048 74 / 60, 2304 89 / 69, 2560 75 / 83, 2816 105 / 86, 4608 125 /
-// 115, and 1.07 or more at every other length up to 40 blocks).
+// 115, and 1.07 or more at every other length up to 40 blocks).  With 6 and 10
+// blocks the walk's lead is 5-10 %, less than a partial round of its larger
+// workgroups costs (1536 columns, 4096 weight rows, n 256 17.4 / 18.4, 320 28.8
+// / 24.3, 512 29.3 / 31.2; 1024 weight rows, n 2553 45.8 / 41.4).
 // Rows too long for the slices' 32-bit offsets (Q6_K from 2^25 columns on) and
 // grids past a launch's 2^32 threads, which the walk's larger tiles reach at
 // twice the size, walk.
@@ -1391,8 +1394,11 @@ bool qmm_slices(int wtype, int rows, int cols, int n) {
     const size_t wgs = qmm_slice_workgroups(rows, n);
     if (qmm_slice_offset(wtype, cols, n) > INT32_MAX || wgs * 512 > UINT32_MAX) return false;
     if (wgs <= 256) return !((wtype == 2 || wtype == 6) && n > 32 && cols > 32 && cols <= 8 * 32);
+    if (wtype != 14) return false;
     const int nb = cols / QK;
-    return wtype == 14 && nb != 1 && !(nb % 4 == 2 && nb <= 10);
+    const size_t walk_wgs = (size_t)((rows + 31) / 32) * (size_t)(qmm_rows_padded(n) / 128);
+    if (nb == 6 || nb == 10) return 2 * ((walk_wgs + 255) / 256) > (wgs + 255) / 256;
+    return nb > 2;
 }
 static bool use_slices(const QmmArgs& a) { return qmm_slices(a.wtype, a.rows, a.cols, a.n); }
 // Activation tiles that the matmul reads.

@@ -187,12 +187,15 @@ def test_qmatmul_slice_offsets_fit_32_bits(lib, wtype, qk, bb):
 
 
 def test_qmatmul_q6k_few_blocks_walk_past_one_round(lib):
-    """Q6_K grids past one workgroup per CU: rows of 1, 2, 6 or 10 blocks take
-    the walking kernel (measured faster there), all others the slices; up to
-    one per CU all take the slices."""
+    """Q6_K grids past one workgroup per CU: rows of 1 or 2 blocks take the
+    walking kernel, and rows of 6 or 10 where its 32 x 128 workgroups need at
+    most half as many rounds as the slices' 32 x 64 (measured faster there);
+    all others the slices, and all up to one workgroup per CU."""
     for nb in range(1, 41):
         assert dr.qmm_plan(14, 4096, 256 * nb, 128)[0]  # 256 workgroups
-        assert dr.qmm_plan(14, 4096, 256 * nb, 129)[0] == (nb not in (1, 2, 6, 10)), nb
+        assert dr.qmm_plan(14, 4096, 256 * nb, 193)[0] == (nb not in (1, 2, 6, 10)), nb  # 256 against 512
+        assert dr.qmm_plan(14, 4096, 256 * nb, 320)[0] == (nb > 2), nb  # 384 against 640
+        assert dr.qmm_plan(14, 1024, 256 * nb, 2553)[0] == (nb > 2), nb  # 640 against 1280
 
 
 @pytest.mark.parametrize("wtype", [2, 6, 8])
