@@ -1031,6 +1031,7 @@ static int qmatmul_impl(dr_ctx* ctx, int wtype, const void* w, size_t rows, size
     a.residual = residual;
     a.norm_w = norm_w;
     a.norm_eps = eps;
+    a.n_cu = ctx->n_cu;
     a.norm_tmp = norm_w ? reinterpret_cast<float*>(static_cast<char*>(ctx->q8k.p) + tmp_off) : nullptr;
     hipError_t e = dr::launch_qmatmul(a, ctx->stream);
     if (e != hipSuccess) return hip_fail(e, "qmatmul launch");
@@ -1767,14 +1768,14 @@ int dr_attention(float* out, size_t out_len, const float* q, size_t q_len, const
 
 long dr_debug_alloc_count(void) { return g_allocs.load(std::memory_order_relaxed); }
 
-int dr_debug_qmm_plan(int wtype, size_t rows, size_t cols, size_t n, int* slices, size_t* max_offset,
+int dr_debug_qmm_plan(int wtype, size_t rows, size_t cols, size_t n, int n_cu, int* slices, size_t* max_offset,
                       size_t* workgroups) {
     size_t qk, bb;
     wtype_block(wtype, qk, bb);
     if (!qk) return fail(DR_ERR_UNSUPPORTED, "dr_debug_qmm_plan: weight type %d not built", wtype);
     if (!slices || !max_offset || !workgroups || !qmm_size_ok(qk, rows, cols, n))
         return fail(DR_ERR_INVALID, "dr_debug_qmm_plan: %zu x %zu x %zu", n, rows, cols);
-    const bool sl = dr::qmm_slices(wtype, (int)rows, (int)cols, (int)n);
+    const bool sl = dr::qmm_slices(wtype, (int)rows, (int)cols, (int)n, n_cu);
     *slices = sl ? 1 : 0;
     *max_offset = sl ? dr::qmm_slice_offset(wtype, (int)cols, (int)n) : 0;
     *workgroups = sl ? dr::qmm_slice_workgroups((int)rows, (int)n)

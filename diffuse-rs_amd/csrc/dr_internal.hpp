@@ -232,6 +232,7 @@ struct QmmArgs {
     const float* norm_w;
     float norm_eps;
     float* norm_tmp;         // with norm_w: [n][rows] f32 for the rows before the norm
+    int n_cu;                // compute units of the device
 };
 
 // The 32-key tiles [kt_lo, kt_hi) that a block of queries at positions
@@ -389,7 +390,7 @@ size_t qmm_workspace_bytes(int n, int cols);
 size_t qmm0_workspace_bytes(int n, int cols);  // the legacy block types
 // dr_qmatmul's kernels: the slices of the blocks (true) or the walk over all
 // of them; the slices' workgroups and the largest 32-bit offset they form.
-bool qmm_slices(int wtype, int rows, int cols, int n);
+bool qmm_slices(int wtype, int rows, int cols, int n, int n_cu);
 size_t qmm_slice_workgroups(int rows, int n);
 size_t qmm_slice_offset(int wtype, int cols, int n);
 hipError_t launch_qmatmul(const QmmArgs& a, hipStream_t st);

@@ -1390,17 +1390,18 @@ size_t qmm_slice_workgroups(int rows, int n) {
 // Rows too long for the slices' 32-bit offsets (Q6_K from 2^25 columns on) and
 // grids past a launch's 2^32 threads, which the walk's larger tiles reach at
 // twice the size, walk.
-bool qmm_slices(int wtype, int rows, int cols, int n) {
+bool qmm_slices(int wtype, int rows, int cols, int n, int n_cu) {
     const size_t wgs = qmm_slice_workgroups(rows, n);
     if (qmm_slice_offset(wtype, cols, n) > INT32_MAX || wgs * 512 > UINT32_MAX) return false;
-    if (wgs <= 256) return !((wtype == 2 || wtype == 6) && n > 32 && cols > 32 && cols <= 8 * 32);
+    const size_t cus = n_cu > 0 ? (size_t)n_cu : 256;
+    if (wgs <= cus) return !((wtype == 2 || wtype == 6) && n > 32 && cols > 32 && cols <= 8 * 32);
     if (wtype != 14) return false;
     const int nb = cols / QK;
     const size_t walk_wgs = (size_t)((rows + 31) / 32) * (size_t)(qmm_rows_padded(n) / 128);
-    if (nb == 6 || nb == 10) return 2 * ((walk_wgs + 255) / 256) > (wgs + 255) / 256;
+    if (nb == 6 || nb == 10) return 2 * ((walk_wgs + cus - 1) / cus) > (wgs + cus - 1) / cus;
     return nb > 2;
 }
-static bool use_slices(const QmmArgs& a) { return qmm_slices(a.wtype, a.rows, a.cols, a.n); }
+static bool use_slices(const QmmArgs& a) { return qmm_slices(a.wtype, a.rows, a.cols, a.n, a.n_cu); }
 // Activation tiles that the matmul reads.
 static int quantized_tiles(const QmmArgs& a) {
     return !use_slices(a) ? a.n_pad / 32 : (a.n <= 32 ? 1 : (a.n + 63) / 64 * 2);

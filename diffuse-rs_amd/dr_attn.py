@@ -178,7 +178,7 @@ _SIGS = {
     "dr_debug_alloc_count": (ctypes.c_long, []),
     "dr_debug_ring_tiles": (_I, [_SZ, _SZ, _SZ, ctypes.c_longlong, ctypes.c_longlong, ctypes.c_longlong, _SZ,
                                  ctypes.POINTER(_I), ctypes.POINTER(_I), ctypes.POINTER(_I)]),
-    "dr_debug_qmm_plan": (_I, [_I, _SZ, _SZ, _SZ, ctypes.POINTER(_I), c_size_p, c_size_p]),
+    "dr_debug_qmm_plan": (_I, [_I, _SZ, _SZ, _SZ, _I, ctypes.POINTER(_I), c_size_p, c_size_p]),
 }
 
 
@@ -658,11 +658,11 @@ def ring_tiles(head_dim: int, nk: int, cap: int, window: Optional[int], qmin: in
     return lo.value, hi.value, bool(ok.value)
 
 
-def qmm_plan(wtype: int, rows: int, cols: int, n: int) -> tuple:
+def qmm_plan(wtype: int, rows: int, cols: int, n: int, n_cu: int = 256) -> tuple:
     """(slices, largest 32-bit offset, workgroups) of dr_qmatmul's kernel for
-    these sizes (dr_debug_qmm_plan); host-only."""
+    these sizes on n_cu compute units (dr_debug_qmm_plan); host-only."""
     sl, off, wgs = ctypes.c_int(), ctypes.c_size_t(), ctypes.c_size_t()
-    _check(load().dr_debug_qmm_plan(wtype, rows, cols, n, ctypes.byref(sl), ctypes.byref(off), ctypes.byref(wgs)))
+    _check(load().dr_debug_qmm_plan(wtype, rows, cols, n, n_cu, ctypes.byref(sl), ctypes.byref(off), ctypes.byref(wgs)))
     return bool(sl.value), off.value, wgs.value
 
 

@@ -196,6 +196,9 @@ def test_qmatmul_q6k_few_blocks_walk_past_one_round(lib):
         assert dr.qmm_plan(14, 4096, 256 * nb, 193)[0] == (nb not in (1, 2, 6, 10)), nb  # 256 against 512
         assert dr.qmm_plan(14, 4096, 256 * nb, 320)[0] == (nb > 2), nb  # 384 against 640
         assert dr.qmm_plan(14, 1024, 256 * nb, 2553)[0] == (nb > 2), nb  # 640 against 1280
+    for wtype in (12, 2, 6, 8):  # the other types: slices up to one workgroup per CU
+        for cus in (64, 256, 304):
+            assert dr.qmm_plan(wtype, 32 * cus, 4096, 64, cus)[0] and not dr.qmm_plan(wtype, 32 * cus + 1, 4096, 64, cus)[0]
 
 
 @pytest.mark.parametrize("wtype", [2, 6, 8])
