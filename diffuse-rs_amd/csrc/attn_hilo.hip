@@ -36,9 +36,10 @@
 // the log2 domain with the lazily moved maximum of the other kernels; l sums
 // the bf16-rounded p that the P.V product multiplies.
 //
-// Head dims 256 and 512 without per-key masks run attn_hilo32_kernel (32-row
-// waves); this kernel takes head dims up to 128, head dims below their tile
-// and MASK_KEYS.
+// attn_hilo32_kernel (32-row waves) takes calls at head dims 256 and 512 with
+// long key loops or a Q epilogue that this kernel would need a pass for; this
+// kernel takes short loops and few rows, head dims up to 128, head dims below
+// their tile and MASK_KEYS (plan_hilo in dr_api.cpp).
 #include "attn_common.hpp"
 
 #include <limits.h>

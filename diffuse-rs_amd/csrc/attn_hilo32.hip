@@ -1,7 +1,8 @@
 // attn_hilo32.hip -- the hi/lo attention (f32-accurate scores and values from
 // bf16 halves, see attn_hilo.hip for the arithmetic) at head dims 256 and 512
 // under position masks (no mask, window, causal prefix, query sequence ids):
-// the layers DiffusionGemma runs at kq_scale 1.0 (forward.rs:338-341).
+// the layers DiffusionGemma runs at kq_scale 1.0 (forward.rs:338-341).  Short
+// key loops without a bias or a rotary stay on the 16-row kernel (plan_hilo).
 //
 // What bounds it.  A hi/lo tile costs 2.5 times the matrix work of a bf16
 // one (three products for the scores, two for the values), and the operands

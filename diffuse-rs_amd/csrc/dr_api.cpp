@@ -1177,20 +1177,19 @@ int dr_cache_initialized(const dr_step_cache* cache, size_t batch) {
 
 // ---------------------------------------------------------------- attention
 
-// The hi/lo kernel's plan: 64 query rows per workgroup, the keys split
-// across workgroups when there are too few of them to fill the chip.
-static dr::LaunchPlan plan_hilo(dr_ctx* ctx, const dr::AttnArgs& a, int hd, int max_nq, int max_nk,
-                                int mask) {
+// The plan of a hi/lo kernel, 16-row or 32-row waves: 64 query rows per
+// workgroup (32-row waves at head dim 256: 128), the keys split across
+// workgroups when there are too few of them to fill the chip.  tiles: key
+// tiles that its busiest CU multiplies.
+static dr::LaunchPlan plan_hilo_rows(dr_ctx* ctx, const dr::AttnArgs& a, int hd_tile, int max_nq, int max_nk,
+                                     int mask, bool w32, int& tiles) {
     dr::LaunchPlan p{};
-    p.hd_tile = hd_tile_for((size_t)hd);
+    p.hd_tile = hd_tile;
     p.block_n = 32;
-    // 32-row waves (attn_hilo32_kernel) at the head dims and masks they are
-    // built for, else the 16-row kernel
-    const bool w32 = dr::hilo32_rows(p.hd_tile) > 0 && hd == p.hd_tile && mask != dr::MASK_KEYS;
-    const int rows = w32 ? dr::hilo32_rows(p.hd_tile) : dr::hilo_rows();
+    const int rows = w32 ? dr::hilo32_rows(hd_tile) : dr::hilo_rows();
     p.rb = rows / 32;
     p.kq = 1;
-    p.waves = !w32 && p.hd_tile > 256 ? 8 : 4;
+    p.waves = !w32 && hd_tile > 256 ? 8 : 4;
     p.stages = 1;
     p.rowgroups = (a.group * max_nq + rows - 1) / rows;
     p.mask = mask;
@@ -1201,7 +1200,7 @@ static dr::LaunchPlan plan_hilo(dr_ctx* ctx, const dr::AttnArgs& a, int hd, int 
     // Workgroups that run at once: the 16-row kernel takes at most 64 KB of
     // LDS up to head dim 256, so two share a CU and key splits fill both; the
     // others take a CU each.
-    const int slots = ctx->n_cu * (w32 || p.hd_tile > 256 ? 1 : 2);
+    const int slots = ctx->n_cu * (w32 || hd_tile > 256 ? 1 : 2);
     int split = 1;
     if (ctx->force_split > 0)
         split = ctx->force_split;
@@ -1209,7 +1208,52 @@ static dr::LaunchPlan plan_hilo(dr_ctx* ctx, const dr::AttnArgs& a, int hd, int 
         split = std::min(slots / std::max(base, 1), ntiles);
     p.n_split = std::max(1, split);
     p.n_workgroups = base * p.n_split;
+    // a workgroup's key range: all keys, or the window around its rows
+    int range = ntiles;
+    if (mask == dr::MASK_POS && a.window >= 0) {
+        const long long near = 2LL * a.window + std::min(max_nq, rows);
+        range = (int)std::min<long long>((a.key_band + 31) / 32, (std::min<long long>(max_nk, near) + 31) / 32 + 1);
+    }
+    tiles = (p.n_workgroups + slots - 1) / slots * ((range + p.n_split - 1) / p.n_split);
     return p;
+}
+
+// 32-row waves (attn_hilo32_kernel) at the head dims and masks they are built
+// for, or the 16-row kernel.  A 32-row tile costs less, a 32-row workgroup
+// starts 2-4 us later and holds the CU alone.
+// - A bias or a full rotary: 32 rows.  They are applied as Q is loaded; the
+//   16-row kernel needs a copy of Q and an epilogue pass first (QK-norm and
+//   RoPE, 16 / 32 rows, us with the store: 16/8 heads of 256, window 1024, 1
+//   row of 65 keys 25 / 21, 64 of 576 41 / 36, 256 of 4352 56 / 46; 16/2 of
+//   512 30 / 22, 53 / 42, 155 / 126).
+// - Else 32 rows where the busiest CU has at least 4 key tiles (shorter
+//   loops do not make up for the later start: 16/8 of 256, 1 row of 65 keys
+//   12 / 15, 64 of 576 25 / 27, 256 of 320 32 / 36, 256 of 4352 66 / 61; 16/2
+//   of 512, 32 of 96 19 / 19, 256 of 4352 126 / 112), where its workgroups
+//   are filled to more than half (8/8 of 256, batch of 4, 2 of 1321 27 / 32;
+//   16/8 of 512, batch of 2, 3 of 4173 58 / 65) and where its larger
+//   workgroups leave no CU with much more to do (16/8 of 256, 659 of 7824,
+//   123 tiles against 82: 225 / 242);
+// - and where the 16-row kernel's second workgroup per CU would leave 48 or
+//   more further splits to merge (8/4 of 256, window 512, 32 of 4128, 128
+//   splits against 64: 36 / 27).
+// (1580 calls without a bias or a rotary, 1-1024 rows, 32-8192 keys, windows
+// and causal prefixes, batches of 1-4: 6 take more than 2 % longer than on the
+// 16-row kernel, 4.7 % at most.)
+static size_t hilo_q_bytes(const dr::AttnArgs& a, const dr::LaunchPlan& p);
+static dr::LaunchPlan plan_hilo(dr_ctx* ctx, const dr::AttnArgs& a, int hd, int max_nq, int max_nk,
+                                int mask) {
+    const int hd_tile = hd_tile_for((size_t)hd);
+    int l16 = 0, l32 = 0;
+    const dr::LaunchPlan p16 = plan_hilo_rows(ctx, a, hd_tile, max_nq, max_nk, mask, false, l16);
+    if (dr::hilo32_rows(hd_tile) == 0 || hd != hd_tile || mask == dr::MASK_KEYS) return p16;
+    const dr::LaunchPlan p32 = plan_hilo_rows(ctx, a, hd_tile, max_nq, max_nk, mask, true, l32);
+    if (hilo_q_bytes(a, p16) > 0 && hilo_q_bytes(a, p32) == 0) return p32;
+    const bool long_loop = l32 >= 4 && 2 * a.group * max_nq >= dr::hilo32_rows(hd_tile) && 20 * l32 <= 27 * l16;
+    // (forced splits: the larger row groups' partials must not outgrow the
+    // fixed scratch of dr_attention_cached_noalloc)
+    const bool fits = dr::split_workspace_bytes(p32, a.n_batch, a.n_head_kv) <= dr::scratch_bytes();
+    return fits && (long_loop || p16.n_split - p32.n_split >= 48) ? p32 : p16;
 }
 
 static dr::LaunchPlan plan_for(dr_ctx* ctx, const dr::AttnArgs& a, int hd, int max_nq,
@@ -1235,7 +1279,8 @@ static dr::LaunchPlan plan_for(dr_ctx* ctx, const dr::AttnArgs& a, int hd, int m
 // full head-dim tile needs none, the kernel applies it as it loads Q (a
 // row's sum of squares over four lanes of one wave, or of the row block's
 // two waves at hd 512).  The 32-row kernel applies all three as it loads Q
-// when the rotary covers the head.
+// when the rotary covers the head; in front of a partial rotary it needs the
+// copy too.
 static size_t hilo_q_bytes(const dr::AttnArgs& a, const dr::LaunchPlan& p) {
     if (p.kernel != dr::KERNEL_HILO || (!a.qn_w && !a.qb && !a.rope)) return 0;
     if (!p.w16 && (!a.rope || a.rot == a.hd)) return 0;
