@@ -597,7 +597,10 @@ __global__ __launch_bounds__(HD) void kv_store_run_kernel(const StoreArgs a) {
             }
         }
     }
-    // the bf16 halves: hi, and lo = bf16 of what that rounding dropped
+    // the bf16 halves: hi, and lo = bf16 of what that rounding dropped (one
+    // turning buffer for both: declared in the lambda, each conversion had its
+    // own, and a hi/lo list workgroup twice the LDS)
+    __shared__ __align__(8) uint16_t s_v[LIST ? HD : 1][VT_KEYS + 4];
     auto put = [&](uint16_t* plane, auto conv) __attribute__((always_inline)) {
         if (!is_v) {
             uint16_t* head = plane + (size_t)g * a.cap * HD + 4 * dc;
@@ -615,7 +618,6 @@ __global__ __launch_bounds__(HD) void kv_store_run_kernel(const StoreArgs a) {
             return;
         }
         if constexpr (LIST) {
-            __shared__ __align__(8) uint16_t s_v[HD][VT_KEYS + 4];
             __syncthreads();  // (the lo plane's turn: the hi values are read)
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
