@@ -16,11 +16,11 @@
 //         ops.rs:384-389, applied before the store in forward.rs:300-302).
 //         A layer kept at hi/lo precision also gets the lo halves,
 //         bf16(x - bf16(x)), of K and V in planes laid out like K and V^T.
-//         One launch.  Rows at contiguous positions (canvas, prompt) or at
-//         a position list: one workgroup per (kv head, 32 rows, K or V),
-//         whole-line loads.  Padded head dims: one workgroup per (64-row
-//         block, 64-wide head-dim chunk, kv head), K converted in registers,
-//         V transposed through LDS.
+//         One launch of one of three kernels (pick_store): one workgroup
+//         per (kv head, 32 rows, K or V) or per (kv head, whole 32-key tile),
+//         whole-line loads; or one per (64-row block, 64-wide head-dim chunk,
+//         kv head), K converted in registers, V transposed through LDS, which
+//         takes padded head dims and unaligned rows too.
 // gather: StepCache::gather (cache.rs:73-82) -- bf16 back to f32 rows (hi +
 //         lo where the layer keeps the lo halves).
 #include <algorithm>
@@ -377,18 +377,29 @@ __global__ __launch_bounds__(256) void kv_store_kernel(const StoreArgs a) {
 }
 
 // The store of rows that fill whole 32-key V^T tiles at contiguous positions
-// (pos0 and n multiples of 32) as they are: no epilogue, no lo halves, head
-// dim == HD (64, 128 or 256).  One workgroup per (kv head, tile) for K and V
-// together; thread (rg, dc), rg fastest, holds the 4 dims 4 dc .. 4 dc + 3
-// of the tile's rows RPG rg .. RPG rg + RPG - 1.  With nothing to compute a
-// step's store is a launch and one round trip, and splitting K from V as
-// kv_store_run_kernel does costs more than it gives (C2's 256 rows of 32
-// heads inside a step: 4.9 against 5.2 us).
+// (pos0 and n multiples of 32), head dim == HD (64, 128 or 256), without lo
+// halves: the canvas rows of every denoise step.  One workgroup per (kv
+// head, tile); thread (rg, dc), rg fastest, holds the 4 dims 4 dc .. 4 dc + 3
+// of the tile's rows RPG rg .. RPG rg + RPG - 1.
+// - Loads: per instruction the wave reads whole 128-byte lines (hd 128: 8
+//   rows x 128 B), against 64-byte pieces at a 64-byte lane stride in
+//   kv_store_kernel.
+// - The K / V biases, the K norm and Gemma's V norm of the epilogue, as in
+//   kv_store_kernel: a row's f32 squares summed in f64, over the 4 dims of
+//   each thread, then across the lanes of the row in the wave (shuffles),
+//   then across the 4 waves in wave order (LDS).  RoPE on K (rotate_rows,
+//   ops.rs:433-452; rot a multiple of 8, so a thread's 4 dims lie on one side
+//   of rot / 2) reads the partner dim d +- rot / 2 of the normed row from LDS
+//   and the (sin, cos) pairs of the row's position, loaded with the rows.
 // - K: bf16 of the 4 dims, 8 bytes per row.
 // - V^T: at step e the thread writes the RPG keys of its rows in d-row
 //   4 dc + e of the tile; the NRG lanes of one dc together write that
 //   d-row's 64 bytes whole, so no LDS transpose and no barrier is needed.
-template <int HD>
+// Same values as kv_store_kernel: bf16 (round to nearest even) of each f32.
+// EPI: the epilogue (biases, norms, RoPE) is compiled in; the plain build
+// keeps it out, since its conditional updates of the loaded rows made the K
+// stores wait for every load.
+template <int HD, bool EPI>
 __global__ __launch_bounds__(256) void kv_store_tiles_kernel(const StoreArgs a) {
     constexpr int CPR = HD / 4;     // 4-dim pieces per row
     constexpr int NRG = 256 / CPR;  // row groups
@@ -411,6 +422,104 @@ __global__ __launch_bounds__(256) void kv_store_tiles_kernel(const StoreArgs a) 
     for (int j = 0; j < RPG; ++j) {
         xk[j] = *reinterpret_cast<const f32x4*>(a.k + src + j * rstride);
         xv[j] = *reinterpret_cast<const f32x4*>(a.v + src + j * rstride);
+    }
+    if constexpr (EPI) {
+        const int half = a.rot / 2;
+        const int d0 = 4 * dc;
+        const bool rot_me = a.rope && d0 < a.rot;
+        f32x4 tab[RPG][2];  // (sin, cos) of pairs jj .. jj + 3 at each row's position
+        if (rot_me) {
+            const int jj = d0 < half ? d0 : d0 - half;
+            const int pp = (a.pos0 >= 0 ? a.pos0 : 0) + r0;
+#pragma unroll
+            for (int j = 0; j < RPG; ++j) {
+                const float* t = a.rope + ((size_t)(pp + j) * half + jj) * 2;
+                tab[j][0] = *reinterpret_cast<const f32x4*>(t);
+                tab[j][1] = *reinterpret_cast<const f32x4*>(t + 4);
+            }
+        }
+        f32x4 kw4 = {}, kb4 = {}, vb4 = {};
+        if (a.kn_w) kw4 = *reinterpret_cast<const f32x4*>(a.kn_w + 4 * dc);
+        if (a.kb) kb4 = *reinterpret_cast<const f32x4*>(a.kb + (size_t)g * HD + 4 * dc);
+        if (a.vb) vb4 = *reinterpret_cast<const f32x4*>(a.vb + (size_t)g * HD + 4 * dc);
+        // (each bias only where given: adding a zero would turn -0.0 into +0.0)
+        if (a.kb) {
+#pragma unroll
+            for (int j = 0; j < RPG; ++j) xk[j] += kb4;
+        }
+        if (a.vb) {
+#pragma unroll
+            for (int j = 0; j < RPG; ++j) xv[j] += vb4;
+        }
+        if (a.kn_w || a.v_norm) {
+            // rms_norm_inplace (ops.rs:106-114) / rms_norm_noscale: sum of the
+            // row's f32 squares in f64; the row's lanes in this wave are lanes
+            // rg + NRG i, the other CPR / (64 / NRG) - 1 shares are in the
+            // other waves
+            __shared__ double s_ss[2][4][VT_KEYS];  // [K, V][wave][row of the tile]
+            const int wave = tid >> 6;
+            auto row_ss = [&](const f32x4 (&x)[RPG], double (&ss)[RPG]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int j = 0; j < RPG; ++j) {
+                    double t = 0.0;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float sq = x[j][e] * x[j][e];
+                        t += (double)sq;
+                    }
+#pragma unroll
+                    for (int off = NRG; off < 64; off <<= 1) t += __shfl_xor(t, off);
+                    ss[j] = t;
+                }
+            };
+            double ssk[RPG], ssv[RPG];
+            if (a.kn_w) row_ss(xk, ssk);
+            if (a.v_norm) row_ss(xv, ssv);
+            if ((tid & 63) < NRG) {
+#pragma unroll
+                for (int j = 0; j < RPG; ++j) {
+                    if (a.kn_w) s_ss[0][wave][rg * RPG + j] = ssk[j];
+                    if (a.v_norm) s_ss[1][wave][rg * RPG + j] = ssv[j];
+                }
+            }
+            __syncthreads();
+            auto scale_of = [&](int kv, int j) __attribute__((always_inline)) {
+                const double t = ((s_ss[kv][0][rg * RPG + j] + s_ss[kv][1][rg * RPG + j]) + s_ss[kv][2][rg * RPG + j]) +
+                                 s_ss[kv][3][rg * RPG + j];
+                return 1.0f / (float)sqrt(t / (double)HD + (double)a.kn_eps);
+            };
+#pragma unroll
+            for (int j = 0; j < RPG; ++j) {
+                if (a.kn_w) {
+                    const float sc = scale_of(0, j);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) xk[j][e] = xk[j][e] * sc * kw4[e];
+                }
+                if (a.v_norm) {
+                    const float sc = scale_of(1, j);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) xv[j][e] *= sc;
+                }
+            }
+        }
+        if (a.rope) {
+            __shared__ __align__(16) float s_k[VT_KEYS][HD + 4];  // the tile's normed K rows
+#pragma unroll
+            for (int j = 0; j < RPG; ++j) *reinterpret_cast<f32x4*>(&s_k[rg * RPG + j][d0]) = xk[j];
+            __syncthreads();
+            if (rot_me) {
+                const int pd0 = d0 < half ? d0 + half : d0 - half;
+#pragma unroll
+                for (int j = 0; j < RPG; ++j) {
+                    const f32x4 xp = *reinterpret_cast<const f32x4*>(&s_k[rg * RPG + j][pd0]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float sn = tab[j][e >> 1][2 * (e & 1)], cs = tab[j][e >> 1][2 * (e & 1) + 1];
+                        xk[j][e] = d0 < half ? rope_lo(xk[j][e], xp[e], sn, cs) : rope_hi(xp[e], xk[j][e], sn, cs);
+                    }
+                }
+            }
+        }
     }
     const int p0 = a.pos0 >= 0 ? a.pos0 : 0;  // (host: pos0 >= 0, or no position list)
     uint16_t* kdst = a.kc + ((size_t)g * a.cap + p0 + r0) * HD + 4 * dc;
@@ -440,9 +549,9 @@ __global__ __launch_bounds__(256) void kv_store_tiles_kernel(const StoreArgs a) 
 }
 
 // The store of rows at contiguous positions or at a sorted position list, head
-// dim == HD: the rows of a denoise step, the prompt, a first pass.  One workgroup per (kv head,
-// 32-key tile that the rows touch, K or V); rows need not fill the first and
-// the last tile.  K and V take a workgroup each, so a step's few tiles give
+// dim == HD: the rows of a denoise step, the prompt, a first pass (pick_store
+// tells which of them).  One workgroup per (kv head, 32-key tile that the rows
+// touch, K or V); rows need not fill the first and the last tile.  K and V take a workgroup each, so a step's few tiles give
 // twice the workgroups, each with half the loads to wait for.
 // Thread (rg, dc), rg fastest, holds keys 4 rg .. 4 rg + 3 of the tile at
 // dims 4 dc .. + 3 and HD / 2 + 4 dc .. + 3.
@@ -458,8 +567,7 @@ __global__ __launch_bounds__(256) void kv_store_tiles_kernel(const StoreArgs a) 
 //   of the wave (shuffles) and the waves in order (LDS).
 // HBM-bound where it is large, latency-bound in a step.  Against the general
 // kernel (64-row blocks, every thread loading the whole row again for the
-// norms), which took runs that fill no whole tiles, hi/lo layers and head dim
-// 512 before: see the figures at launch_store.
+// norms) and the tile kernel: see the figures at pick_store.
 // EPI: biases, norms and RoPE are compiled in (the plain build keeps them
 // out: its stores then wait for their own loads only).  HILO: the lo planes
 // are written too.  LIST: the rows go to the positions of a sorted list
@@ -693,6 +801,80 @@ void launch_run(const StoreArgs& a, bool epi, dim3 grid, hipStream_t st) {
     }
 }
 
+enum StoreKernel { STORE_GENERAL, STORE_RUN, STORE_TILES };
+
+// The kernel of a store.  The run kernel takes every call whose head dim fills
+// its tile, the tile kernel whole 32-key tiles of bf16 layers up to head dim
+// 256; the general kernel takes all.  g: (kv head, 32 rows) pairs, as many as
+// the tile kernel has workgroups, per 256 CUs (a batch slot's store has only
+// its XCDs); the run kernel has twice as many, of half the work each.  So up
+// to 128 it fills CUs that the others leave idle, and past that its second
+// load of the epilogue's operands and its half-rows of DRAM traffic count.
+// us, heads x head dim:
+// - with RoPE, not whole bf16 tiles: run (general / run: 16 x 128, 512 rows
+//   from position 517, norm + RoPE 12.6 / 5.7; hi/lo 8 x 256, 4352 rows 97 / 35;
+//   2 x 512, 256 rows 12.8 / 8.7; 32 x 128, 145 listed rows 10.3 / 5.3).
+// - norms or biases alone, the same: run, but for hi/lo layers and lists at
+//   head dim 512 with up to 64 pairs, where the general kernel's 64-wide
+//   pieces fill more CUs (K norm, hi/lo, 256 rows of 2 x 512 7.8 / 9.3, 1536
+//   17.4 / 11.0; rows past whole 64s cost it a second pass: 145 14.6 / 9.2).
+// - nothing to compute: contiguous rows, run (32 x 128, 256 rows 7.1 / 5.1),
+//   but for a few rows of a hi/lo layer (8 x 256, 32 rows 5.4 / 5.8, 64 6.2 /
+//   5.8).  Lists and hi/lo tiles: at head dims 64 and 128 run up to the pairs
+//   where the chip is full (list: 32 x 128, 128 rows 4.2 / 3.8, 512 7.1 / 8.5,
+//   1024 14.3 / 13.5; hi/lo 512 10.5 / 12.6, 1024 18.8 / 19.1; 12 x 64, 512
+//   4.0 / 3.5, 2560 6.8 / 8.0), at 256 and 512 the general kernel's pieces
+//   until they fill it (list: 8 x 256, 145 4.1 / 4.7, 1536 12.3 / 11.8; hi/lo
+//   tiles: 2 x 512, 256 4.3 / 6.4, 8 x 512, 512 9.1 / 8.9).
+// - whole bf16 tiles with an epilogue, tile / run: partial rotaries turn
+//   through LDS on both, tile (16 x 128, 256 rows 4.2 / 4.5, 1024 6.7 / 8.8; 8
+//   x 256 6.4 / 5.9 at 512, 7.3 / 8.7 at 1024; with a norm at 256 9.9 / 7.5);
+//   head dim 64 (a wave's 8 rows in run are 2 KB): tile (8 x 64, K norm, 256
+//   3.5 / 4.2), but for a full rotary without a lone K norm (RoPE 3.4 / 3.3 at
+//   256, 3.6 / 3.8 at 768, 4.7 / 4.5 at 1536); head dim 128: run while it
+//   fills idle CUs (16 x 128, K norm 5.1 / 4.7 at 256, 7.0 / 7.3 at 1024; bias +
+//   RoPE 5.3 / 4.2, 17.1 / 17.7 at 2560; norm + RoPE 6.5 / 5.2, 18.5 / 19.0),
+//   always with the V norm (two norms in one thread: 14.0 / 11.9 at 1536); head
+//   dim 256: run (8 x 256, norm + RoPE 10.9 / 6.3 at 256, 35.9 / 29.4 at 4352),
+//   but for biases alone past 128 pairs (16 x 256, 1024 10.5 / 12.9).
+StoreKernel pick_store(int hd_tile, const StoreArgs& a, int p0, bool epi) {
+    const bool partial = a.rope && a.rot != a.hd;
+    const bool run = a.vec && a.hd == hd_tile && !a.klo == !a.vlo &&
+                     (!partial || (hd_tile <= 256 && a.rot % 8 == 0 && a.rot <= a.hd)) &&
+                     (((uintptr_t)a.kn_w | (uintptr_t)a.kb | (uintptr_t)a.vb | (uintptr_t)a.rope) & 15) == 0;
+    if (!run) return STORE_GENERAL;
+    const bool hilo = a.klo != nullptr, list = p0 < 0, kn = a.kn_w != nullptr, vn = a.v_norm != 0;
+    const bool whole = !list && p0 % VT_KEYS == 0 && a.n % VT_KEYS == 0;
+    const long g = (long)a.n_head_kv * ((a.n + VT_KEYS - 1) / VT_KEYS) * 8 / a.xcd_n;
+    if (whole && !hilo && hd_tile <= 256) {
+        bool tiles;
+        if (!epi)
+            tiles = true;
+        else if (hd_tile == 64)
+            tiles = !a.rope || partial || (kn && !vn) || (g > 128 && g <= 256) || g >= 1024;
+        else if (partial)
+            tiles = hd_tile == 128 || (!kn && !vn && g > 128);
+        else if (!a.rope && !vn && !(kn && hd_tile == 256))
+            tiles = g > 128;
+        else
+            tiles = hd_tile == 128 && !vn && g >= (kn || a.n_head_kv < 16 ? 1024 : 512);
+        return tiles ? STORE_TILES : STORE_RUN;
+    }
+    bool general;
+    if (epi)
+        general = hd_tile == 512 && !a.rope && !vn && g <= 64 && (hilo ? list || whole : list && !kn) &&
+                  (!kn || a.n % SR == 0);
+    else if (!list && !whole)
+        general = hilo && a.n <= (hd_tile >= 256 ? hd_tile / 8 : 4);
+    else if (hd_tile == 64)
+        general = g > (hilo ? 320 : 640);
+    else if (hd_tile == 128)
+        general = g > 128 && (hilo || g < 1024);
+    else
+        general = g <= (hd_tile == 256 ? (list ? 320 : 128) : (list ? 192 : 64)) && (hilo || whole || a.n >= VT_KEYS);
+    return general ? STORE_GENERAL : STORE_RUN;
+}
+
 }  // namespace
 
 hipError_t launch_store(int hd_tile, const StoreArgs& args, hipStream_t st) {
@@ -706,39 +888,25 @@ hipError_t launch_store(int hd_tile, const StoreArgs& args, hipStream_t st) {
     const int nb = a.n_batch > 0 ? a.n_batch : 1;
     a.xcd_lo = 8 * a.batch / nb;
     a.xcd_n = std::max(1, 8 * (a.batch + 1) / nb - a.xcd_lo);
-    // Rows at contiguous positions whose head dim fills its tile: the tile
-    // kernel where they are whole tiles to be stored as they are, else the
-    // run kernel, which also takes position lists.  Padded head dims, rows that
-    // are not 16-byte aligned and a partial rotary at head dim 512 take the
-    // general kernel.
-    // Run kernel against the kernels that took these calls before (general;
-    // * the tile kernel with an epilogue), in us, kernel times:
-    //   16 heads, hd 128, 512 rows from position 2041, norm + RoPE   12.5 / 7.0
-    //   8 heads, hd 256, 256 rows, hi/lo, norms + RoPE               11.9 / 7.7
-    //   2 heads, hd 512, 256 rows, hi/lo, norms + RoPE               20.7 / 12.3
-    //   8 heads, hd 256, 4352 rows, hi/lo, norms + RoPE               121 / 47.7
-    //   4 heads, hd 128, 1280 rows, bias + RoPE *                     7.8 / 6.5
-    //   32 heads, hd 128, 64 rows, RoPE *                             5.1 / 4.0
-    //   32 heads, hd 128, 145 listed rows of 256 positions, RoPE      8.2 / 5.6
-    //   the same, 404 of 512                                         12.1 / 9.0
     const int p0 = a.pos0 >= 0 ? a.pos0 : (a.pos == nullptr ? 0 : -1);
-    const bool rot_ok = !a.rope || a.rot == a.hd || (hd_tile <= 256 && a.rot % 8 == 0 && a.rot <= a.hd);
-    const bool run = a.vec && a.hd == hd_tile && rot_ok && !a.klo == !a.vlo &&
-                     (((uintptr_t)a.kn_w | (uintptr_t)a.kb | (uintptr_t)a.vb | (uintptr_t)a.rope) & 15) == 0;
     const bool epi = a.kn_w || a.kb || a.vb || a.v_norm || a.rope;
-    if (run && p0 >= 0 && !epi && !a.klo && hd_tile <= 256 && p0 % VT_KEYS == 0 && a.n % VT_KEYS == 0) {
+    const StoreKernel kernel = pick_store(hd_tile, a, p0, epi);
+    if (kernel == STORE_TILES) {
         a.pos0 = p0;
         const int work = a.n_head_kv * (a.n / VT_KEYS);
         a.per_xcd = (work + a.xcd_n - 1) / a.xcd_n;
         const dim3 grid((unsigned)(8 * a.per_xcd));
-        switch (hd_tile) {
-            case 64: hipLaunchKernelGGL(kv_store_tiles_kernel<64>, grid, dim3(256), 0, st, a); break;
-            case 128: hipLaunchKernelGGL(kv_store_tiles_kernel<128>, grid, dim3(256), 0, st, a); break;
-            default: hipLaunchKernelGGL(kv_store_tiles_kernel<256>, grid, dim3(256), 0, st, a); break;
+        switch (hd_tile * 2 + (epi ? 1 : 0)) {
+            case 128: hipLaunchKernelGGL((kv_store_tiles_kernel<64, false>), grid, dim3(256), 0, st, a); break;
+            case 129: hipLaunchKernelGGL((kv_store_tiles_kernel<64, true>), grid, dim3(256), 0, st, a); break;
+            case 256: hipLaunchKernelGGL((kv_store_tiles_kernel<128, false>), grid, dim3(256), 0, st, a); break;
+            case 257: hipLaunchKernelGGL((kv_store_tiles_kernel<128, true>), grid, dim3(256), 0, st, a); break;
+            case 512: hipLaunchKernelGGL((kv_store_tiles_kernel<256, false>), grid, dim3(256), 0, st, a); break;
+            default: hipLaunchKernelGGL((kv_store_tiles_kernel<256, true>), grid, dim3(256), 0, st, a); break;
         }
         return hipGetLastError();
     }
-    if (run) {
+    if (kernel == STORE_RUN) {
         const bool list = p0 < 0;
         a.pos0 = p0;
         a.n_rb = list ? (a.n + VT_KEYS - 1) / VT_KEYS : (p0 + a.n - 1) / VT_KEYS - p0 / VT_KEYS + 1;

@@ -48,7 +48,33 @@ def test_store_list_vs_oracle(dev, hd, hkv, n, epi, rot, hilo):
     _store_and_check(dev, hd, hkv, sorted(rng.choice(3 * n + 40, n, replace=False).tolist()), epi, rot, hilo)
 
 
-def _store_and_check(dev, hd, hkv, positions, epi, rot, hilo):
+@pytest.mark.parametrize("hd,hkv,p0,n,ops,rot,hilo", [
+    # whole tiles of bf16 layers with an epilogue, both sides of the rule between the tile and the run kernel
+    (64, 2, 32, 64, "n", 0, False), (64, 2, 0, 96, "b", 24, False), (64, 3, 32, 32, "b", 64, False),
+    (64, 8, 0, 32 * 17, "", 64, False), (64, 8, 64, 32 * 33, "nv", 64, False), (128, 2, 64, 64, "bn", 64, False),
+    (128, 8, 32, 32 * 16, "b", 0, False), (128, 8, 0, 32 * 17, "b", 0, False), (128, 8, 0, 32 * 17, "n", 128, False),
+    (128, 16, 0, 32 * 32, "b", 128, False), (128, 16, 0, 32 * 64, "n", 128, False), (128, 4, 0, 96, "v", 0, False),
+    (256, 2, 32, 64, "n", 256, False), (256, 8, 0, 32 * 17, "b", 0, False), (256, 8, 0, 32 * 17, "", 64, False),
+    (256, 2, 32, 64, "nv", 64, False),
+    # hi/lo tiles and head dim 512, both sides of the rule between the general and the run kernel
+    (64, 8, 0, 32 * 41, "", 0, True), (128, 8, 0, 32 * 17, "", 0, True), (256, 8, 0, 32 * 16, "", 0, True),
+    (256, 8, 0, 32 * 17, "", 0, True), (512, 2, 0, 64, "n", 0, True), (512, 2, 0, 96, "n", 0, True),
+    (512, 2, 32, 64, "b", 0, True), (512, 2, 64, 32 * 33, "", 0, False), (256, 2, 5, 20, "", 0, True),
+])
+def test_store_whole_tiles_vs_oracle(dev, hd, hkv, p0, n, ops, rot, hilo):
+    _store_and_check(dev, hd, hkv, list(range(p0, p0 + n)), bool(ops or rot), rot, hilo, ops)
+
+
+@pytest.mark.parametrize("hd,hkv,n,hilo", [
+    (64, 8, 32 * 81, False), (64, 8, 32 * 41, True), (128, 8, 32 * 17, False), (128, 8, 32 * 17, True),
+    (256, 2, 31, False), (256, 8, 32 * 40, True), (256, 8, 32 * 41, True), (512, 2, 70, True), (512, 4, 32 * 49, False),
+])
+def test_store_plain_lists_both_sides(dev, hd, hkv, n, hilo):
+    rng = np.random.default_rng(hd + n)
+    _store_and_check(dev, hd, hkv, sorted(rng.choice(2 * n + 40, n, replace=False).tolist()), False, 0, hilo)
+
+
+def _store_and_check(dev, hd, hkv, positions, epi, rot, hilo, ops="bnv"):
     n = len(positions)
     rng = np.random.default_rng(hd + positions[0] + 3 * n + rot)
     n_t, kvs, eps, put = positions[-1] + 36, hkv * hd, 1e-6, dev.put
@@ -60,19 +86,24 @@ def _store_and_check(dev, hd, hkv, positions, epi, rot, hilo):
     if epi:
         bk, bv = ((0.1 * rng.standard_normal(kvs)).astype(np.float32) for _ in range(2))
         kn = rng.uniform(0.5, 1.5, hd).astype(np.float32)
+        kw = dict(bk=put(bk), bv=put(bv)) if "b" in ops else {}
+        if "n" in ops:
+            kw.update(k_norm_w=put(kn))
         q = np.zeros(n * kvs, np.float32)
-        cache.step_epi(0, [(put(q), dev.empty(n * kvs), p, put(K), put(V))], hkv, scale=1 / math.sqrt(hd), bk=put(bk),
-                       bv=put(bv), k_norm_w=put(kn), v_norm=True, eps=eps,
-                       rope=dr.Rope(dev.ctx, n_t, rot, 10000.0) if rot else None)
-        orc.add_bias(wk, bk, n)
-        orc.add_bias(wv, bv, n)
+        cache.step_epi(0, [(put(q), dev.empty(n * kvs), p, put(K), put(V))], hkv, scale=1 / math.sqrt(hd), v_norm="v" in ops,
+                       eps=eps, rope=dr.Rope(dev.ctx, n_t, rot, 10000.0) if rot else None, **kw)
+        if "b" in ops:
+            orc.add_bias(wk, bk, n)
+            orc.add_bias(wv, bv, n)
         for o in range(0, wk.size, hd):
-            seg = wk[o:o + hd].copy()
-            orc.rms_norm_inplace(seg, kn, eps)
-            wk[o:o + hd] = seg
-            seg = wv[o:o + hd].copy()
-            orc.rms_norm_noscale(seg, eps)
-            wv[o:o + hd] = seg
+            if "n" in ops:
+                seg = wk[o:o + hd].copy()
+                orc.rms_norm_inplace(seg, kn, eps)
+                wk[o:o + hd] = seg
+            if "v" in ops:
+                seg = wv[o:o + hd].copy()
+                orc.rms_norm_noscale(seg, eps)
+                wv[o:o + hd] = seg
         if rot:
             orc.rotate_rows(wk, orc.rope_table(n_t, rot, 10000.0), positions, hkv, hd, rot)
     else:
