@@ -198,8 +198,9 @@ def test_hilo_gather_returns_hi_plus_lo(dev):
 
 def test_hilo_step_epi_vs_oracle(dev):
     """dr_attention_step_epi on a hi/lo layer: the Q epilogue (bias, QK-norm,
-    RoPE) runs on a copy of Q before the hi/lo kernel; K's lo half is taken
-    after the K epilogue.  Gemma-like: V-norm, window, scale 1.0."""
+    RoPE) is applied as the 32-row hi/lo kernel loads Q (test_gpu_hilo_qcopy.py
+    has the calls that run it on a copy); K's lo half is taken after the K
+    epilogue.  Gemma-like: V-norm, window, scale 1.0."""
     h, hkv, hd, rot, n_p, n_c, window = 8, 4, 256, 256, 300, 120, 128
     rng = np.random.default_rng(2561)
     eps = 1e-6

@@ -71,3 +71,45 @@ def test_rows_kernel_vs_oracle(dev, name):
     assert (info["kernel"], info["waves_per_wg"], info["row_blocks"], info["key_groups"]) == (dr.KERNEL_STAGED, 4, 2, 2)
     for b in range(batch):
         check(dev.get(items[b][1]), wants[b], f"{name} slot {b}")
+
+
+@pytest.mark.parametrize("h,hkv,hd,n_t,slots,window,prefix", [
+    (48, 48, 64, 333, (range(333), range(301, 333), [7, 64, 65, 332]), None, 300),
+    (84, 12, 128, 150, (range(100, 150), range(150), [0, 149]), 40, None),
+])
+def test_rows_kernel_slots_of_different_lengths(dev, h, hkv, hd, n_t, slots, window, prefix):
+    """Batch slots of different lengths (the shorter ones' workgroups past
+    their rows leave at once) in rows of a fused QKV projection, with the
+    whole Q epilogue."""
+    rng = np.random.default_rng(h + hd)
+    qs, kvs, eps, put, scale = h * hd, hkv * hd, 1e-6, dev.put, 1 / math.sqrt(hd)
+    fused = qs + 2 * kvs
+    qn, kn = (rng.uniform(0.5, 1.5, hd).astype(np.float32) for _ in range(2))
+    bq, bk, bv = ((0.1 * rng.standard_normal(m)).astype(np.float32) for m in (qs, kvs, kvs))
+    table = orc.rope_table(n_t, hd, 10000.0)
+    cache = dr.StepCache(dev.ctx, n_t, [hkv], [hd], n_batch=len(slots))
+    items, wants, keep = [], [], []
+    for b, active in enumerate(map(list, slots)):
+        n = len(active)
+        K, V = (rng.standard_normal((n_t, kvs)).astype(np.float32) for _ in range(2))
+        R = rng.standard_normal((n, fused)).astype(np.float32)
+        cache.store(0, dr.Pass(dev.ctx, range(n_t)), put(K), put(V), batch=b)
+        rows, out = put(R), dev.empty(n * qs)
+        base = rows.data_ptr()
+        items.append((base, out, dr.Pass(dev.ctx, active), base + 4 * qs, base + 4 * (qs + kvs)))
+        keep.append((rows, out))
+        q, k, v = _epilogue_oracle(R[:, :qs].reshape(-1).copy(), R[:, qs:qs + kvs].reshape(-1).copy(),
+                                   R[:, qs + kvs:].reshape(-1).copy(), active, h, hkv, hd, bq, bk, bv, qn, kn, False,
+                                   eps, table, hd)
+        K[active], V[active] = k.reshape(n, kvs), v.reshape(n, kvs)
+        s = Shape(n, n_t, h, hkv, hd, sliding_window=window, causal_prefix=prefix, scale=scale)
+        c = np.float32(scale * 1.4426950408889634)
+        wants.append(oracle_run(s, RowsSpec(active), RowsSpec(list(range(n_t))), bf16_round(q * c) / c,
+                                bf16_round(K.reshape(-1)), bf16_round(V.reshape(-1))))
+    cache.step_rows(0, items, h, fused, fused, sliding_window=window, causal_prefix=prefix, scale=scale, bq=put(bq),
+                    bk=put(bk), bv=put(bv), q_norm_w=put(qn), k_norm_w=put(kn), eps=eps,
+                    rope=dr.Rope(dev.ctx, n_t, hd, 10000.0))
+    info = dev.ctx.last_launch()
+    assert (info["kernel"], info["waves_per_wg"], info["row_blocks"], info["key_groups"]) == (dr.KERNEL_STAGED, 4, 2, 2)
+    for b, (_, out) in enumerate(keep):
+        check(dev.get(out), wants[b], f"slot {b}")
