@@ -5,8 +5,8 @@ epilogue).  Read in place through row strides, the step must give the same
 bits -- outputs and cache contents -- as dr_attention_step_epi on the copied
 Q, K and V, on every path the strides touch: the per-wave-stream kernel's Q
 load with the folded epilogue, the staged kernel's (partial rotary), the
-hi/lo kernel's Q copy, the whole-tile store and the position-list store, two
-batch slots.  Needs an MI355X.
+32-row hi/lo kernel's (the hi/lo layers' Q copy: test_gpu_hilo_qcopy.py), the
+whole-tile store and the position-list store, two batch slots.  Needs an MI355X.
 """
 from __future__ import annotations
 
