@@ -15,7 +15,7 @@ import pytest
 
 import dr_attn as dr
 import oracle as orc
-from helpers import RowsSpec, Shape
+from helpers import RowsSpec, Shape, brute_force
 
 from test_gpu_parity import _epilogue_oracle, check, dev, oracle_run, say, torch  # noqa: F401
 
@@ -166,3 +166,32 @@ def test_hilo_forced_splits_fit_the_fixed_scratch(dev):
     assert info["n_split"] == 32 and info["rows_per_wave"] == 16
     s = Shape(n, n_t, h, h, hd, scale=1.0)
     check(dev.get(out), oracle_run(s, RowsSpec(active), RowsSpec(list(range(n_t))), Q, K, V), "32 forced splits")
+
+
+def test_hilo32_error_against_64_bits(dev):
+    """Near one-hot rows at scale 1.0, 64 rows over one range of 32 key tiles:
+    a row's largest weight is exactly 1 in bf16 (the running maximum is its
+    score), so only the others' rounding reaches the output: 2.5e-4 here,
+    4.3e-4 when the maximum moves only past a threshold of 8.  Bound between
+    them, at their geometric mean."""
+    h, hd, n_t, n = 4, 256, 1024, 64
+    rng = np.random.default_rng(256)
+    K, V = (rng.standard_normal(n_t * h * hd).astype(np.float32) for _ in range(2))
+    Q = rng.standard_normal(n * h * hd).astype(np.float32)
+    active = list(range(n_t - n, n_t))
+    cache = dr.StepCache(dev.ctx, n_t, [h], [hd], precision=[dr.PRECISION_HILO])
+    cache.store(0, dr.Pass(dev.ctx, range(n_t)), dev.put(K), dev.put(V))
+    rows = slice((n_t - n) * h * hd, None)
+    out = dev.empty(n * h * hd)
+    dev.ctx.set_split(1)
+    try:  # (a bias, of zeros: the 32-row kernel)
+        cache.step_epi(0, [(dev.put(Q), out, dr.Pass(dev.ctx, active), dev.put(K[rows].copy()), dev.put(V[rows].copy()))],
+                       h, scale=1.0, bq=dev.put(np.zeros(h * hd, np.float32)))
+        info = dev.ctx.last_launch()
+    finally:
+        dev.ctx.set_split(0)
+    assert info["rows_per_wave"] == 32 and info["n_split"] == 1
+    want = brute_force(Q, K, V, Shape(n, n_t, h, h, hd, scale=1.0), RowsSpec(active), RowsSpec(list(range(n_t))))
+    err = np.linalg.norm(dev.get(out).reshape(want.shape) - want) / np.linalg.norm(want)
+    say(f"relative error {err:.3e}")
+    assert err < 3.3e-4
