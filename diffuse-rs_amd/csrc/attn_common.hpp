@@ -253,5 +253,22 @@ __device__ __forceinline__ float2 load2_sc1(__amdgpu_buffer_rsrc_t r, int voff) 
     return make_float2(__uint_as_float(v[0]), __uint_as_float(v[1]));
 }
 
+// 16 bytes per lane, buffer -> LDS, at LDS byte address `lds` + 16 * lane.
+// As inline asm (attn_rows.hip, attn_hilo32.hip; it has no outputs): the
+// compiler would make every later LDS read wait for the DMA, since it cannot tell
+// the buffers apart.  The kernels' own waits order them.  (M0 needs one wait state before the load;
+// the kernels make no other use of M0, which the compiler cannot be told is
+// clobbered.)
+__device__ __forceinline__ void dma16_asm(__amdgpu_buffer_rsrc_t r, uint32_t lds, int voff, int soff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds),
+        "v"(voff), "s"(r), "s"(soff)
+        : "memory");
+#endif
+}
+
 }  // namespace
 }  // namespace dr

@@ -74,23 +74,6 @@ struct Hilo32Geom {
     static_assert(LDS_BYTES <= 159 * 1024, "LDS budget");
 };
 
-// 16 bytes per lane, buffer -> LDS, at LDS byte address `lds` + 16 * lane.
-// As inline asm (it has no outputs): the compiler would make every later LDS
-// read wait for the DMA, since it cannot tell the buffers apart.  The
-// kernel's own waits order them.  (M0 needs one wait state before the load;
-// the kernel makes no other use of M0, which the compiler cannot be told is
-// clobbered.)
-__device__ __forceinline__ void dma16_asm(__amdgpu_buffer_rsrc_t r, uint32_t lds, int voff, int soff) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile(
-        "s_mov_b32 m0, %0\n\t"
-        "s_nop 0\n\t"
-        "buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds),
-        "v"(voff), "s"(r), "s"(soff)
-        : "memory");
-#endif
-}
-
 // a + (16 lanes away) in the even rows of 16 lanes, b + the same in the odd
 // ones
 __device__ __forceinline__ double swap_add16(double a, double b) {

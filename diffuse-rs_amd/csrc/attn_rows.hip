@@ -58,19 +58,6 @@ struct RowsGeom {
     static_assert(DMAW >= 1, "DMA split");
 };
 
-// (see attn_hilo32.hip: the compiler would make every LDS read wait for a
-// DMA it knows of)
-__device__ __forceinline__ void dma16_asm(__amdgpu_buffer_rsrc_t r, uint32_t lds, int voff, int soff) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile(
-        "s_mov_b32 m0, %0\n\t"
-        "s_nop 0\n\t"
-        "buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds),
-        "v"(voff), "s"(r), "s"(soff)
-        : "memory");
-#endif
-}
-
 // maximum of a lane and its partner lane ^ 32
 __device__ __forceinline__ float max_xor32(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
