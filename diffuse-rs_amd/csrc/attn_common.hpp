@@ -1,5 +1,6 @@
 // attn_common.hpp -- device helpers shared by the attention kernels
-// (attn_fwd.hip, attn_ring.hip): vector types, the LDS tile swizzle and key
+// (attn_fwd.hip, attn_ring.hip, attn_rows.hip, attn_hilo.hip,
+// attn_hilo32.hip): vector types, the LDS tile swizzle and key
 // permutations of the 32-key K tiles, LDS-DMA, visible() of attention.rs:36-57,
 // and the packed-row decode of GQA query rows.
 #pragma once
@@ -255,10 +256,10 @@ __device__ __forceinline__ float2 load2_sc1(__amdgpu_buffer_rsrc_t r, int voff) 
 
 // 16 bytes per lane, buffer -> LDS, at LDS byte address `lds` + 16 * lane.
 // As inline asm (attn_rows.hip, attn_hilo32.hip; it has no outputs): the
-// compiler would make every later LDS read wait for the DMA, since it cannot tell
-// the buffers apart.  The kernels' own waits order them.  (M0 needs one wait state before the load;
-// the kernels make no other use of M0, which the compiler cannot be told is
-// clobbered.)
+// compiler would make every later LDS read wait for the DMA, since it cannot
+// tell the buffers apart.  The kernels' own waits order them.  (M0 needs one
+// wait state before the load; the kernels make no other use of M0, which the
+// compiler cannot be told is clobbered.)
 __device__ __forceinline__ void dma16_asm(__amdgpu_buffer_rsrc_t r, uint32_t lds, int voff, int soff) {
 #if defined(__HIP_DEVICE_COMPILE__)
     asm volatile(

@@ -1614,8 +1614,12 @@ LaunchPlan plan_attention(int hd, int n_batch, int n_head_kv, int group, int max
     // store, us, staged / rows (workgroups): Dream 2 x 1280 first pass 107 / 92
     // (1120), 4 x 256 of 1280 54.3 / 49.9 (448); 32 heads 2560 first pass 193
     // / 163 (1280), 768 first pass 40.6 / 36.2 (384), 4 x 256 of 768 88 / 82
-    // (512); 8/2 heads of 64, 2 x 4000 first pass 132 / 100 (1000).  At or
-    // below one per CU the staged kernel's 8 waves win: 16 heads 1000 first
+    // (512); 8/2 heads of 64, 2 x 4000 first pass 132 / 100 (1000).  Just past
+    // one per CU and under windows too: 16 heads, window 1024, 1083 rows of
+    // 3131 keys 42.7 / 37.7 (272) and, 18 row groups a head, 43.4 / 38.1 (288);
+    // over 582 random calls of 257-704 workgroups, plain, windowed and causal,
+    // the staged kernel took 1.13 times as long at the least and 1.45 in the
+    // median.  At or below one per CU the staged kernel's 8 waves win: 16 heads 1000 first
     // pass 30.9 / 31.3 (256), 2 x 256 of 768 32.3 / 33.2 (256), 8/2 heads of
     // 64 2000 first pass 24.4 / 26.0 (250), Dream 2 x 256 of 1280 28.9 / 31.6
     // (224).  Workgroups of 128 rows (half the K/V stream) lose to their

@@ -4,10 +4,14 @@
 // MASK_POS (window, causal prefix, query sequence ids), with the whole Q
 // epilogue.
 //
-// What bounds it.  With rows to fill the chip several times over, the matrix
-// cores: a copy of this kernel without softmax, LDS reads and DMA still takes
-// 60 % of its time, at 1095 TFLOP/s (a 8192^3 bf16 product reaches 1280 on
-// the card).  DMA and the return of its lines cost 15 %, the VALU 8 %.  The
+// What bounds it.  With rows to fill the chip several times over (32 heads,
+// 2560 rows), the matrix cores: a copy of this kernel without softmax, LDS
+// reads and DMA still takes 60 % of its time, at 1095 TFLOP/s (a 8192^3 bf16
+// product reaches 1280 on the card); DMA and the return of its lines cost
+// 15 %, the VALU 8 %.  At 28/4 heads, 2 x 1280 rows (1120 workgroups, little
+// over two rounds) the matrix cores are busy 30 % of the CUs' busy time and
+// the texture data path, which returns the DMA's lines, 72 % of the call; no
+// LDS bank conflicts, 91 % of the lines from L2.  The
 // staged kernel's 64-row workgroups of 8 waves (4 key groups of one tile
 // each) pass a workgroup barrier per super-tile with a tile's scores, softmax
 // and values in sequence.  Here a workgroup is 4 waves, two row blocks of 32

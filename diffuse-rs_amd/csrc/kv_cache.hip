@@ -551,8 +551,9 @@ __global__ __launch_bounds__(256) void kv_store_tiles_kernel(const StoreArgs a) 
 // The store of rows at contiguous positions or at a sorted position list, head
 // dim == HD: the rows of a denoise step, the prompt, a first pass (pick_store
 // tells which of them).  One workgroup per (kv head, 32-key tile that the rows
-// touch, K or V); rows need not fill the first and the last tile.  K and V take a workgroup each, so a step's few tiles give
-// twice the workgroups, each with half the loads to wait for.
+// touch, K or V); rows need not fill the first and the last tile.  K and V
+// take a workgroup each, so a step's few tiles give twice the workgroups, each
+// with half the loads to wait for.
 // Thread (rg, dc), rg fastest, holds keys 4 rg .. 4 rg + 3 of the tile at
 // dims 4 dc .. + 3 and HD / 2 + 4 dc .. + 3.
 // - Loads: an instruction reads 8 rows x 128 bytes, whole lines.

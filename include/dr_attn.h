@@ -546,10 +546,10 @@ int dr_debug_ring_tiles(size_t head_dim, size_t nk, size_t cap, long long window
                         long long qmax, size_t n_split, int* min_tile, int* max_tile,
                         int* partition_ok);
 /* The kernel family that dr_qmatmul runs for these sizes on a device of n_cu
- * compute units: slices (1), where
- * each wave takes an eighth of a row's blocks, or the walk over all blocks
- * (0); its workgroups of 512 threads; and with slices the largest byte offset
- * that its 32-bit offsets have to hold.  Host-only. */
+ * compute units: slices (1), where each wave takes an eighth of a row's
+ * blocks, or the walk over all blocks (0); its workgroups of 512 threads; and
+ * with slices the largest byte offset that its 32-bit offsets have to hold.
+ * Host-only. */
 int dr_debug_qmm_plan(int wtype, size_t rows, size_t cols, size_t n, int n_cu, int* slices, size_t* max_offset,
                       size_t* workgroups);
 
